@@ -230,3 +230,18 @@ def test_model_io_host_validation():
     assert "grid dtype" in _err(h.wam_rope_freqs(ctypes.byref(f), None))
     f.grid_dtype, f.head_dim = _lib.WAM_I64, 130
     assert "whole f/h/w pairs" in _err(h.wam_rope_freqs(ctypes.byref(f), None))
+
+
+def test_small_grid_plan_workspace():
+    """Few rows: whole k ranges of fp32 partial sums, at most one per k-tile
+    and 32, for every segment; none where one round of tiles covers the chip."""
+    h = _lib.lib()
+    for M in (1, 16, 32, 33, 64, 65, 128, 224, 300, 780, 1024, 2325):
+        for N, n_seg, K in ((3072, 1, 3072), (3072, 3, 3072), (14336, 1, 3072), (3072, 1, 14336), (1536, 2, 64),
+                            (192, 1, 3072), (200, 1, 192)):
+            n = h.wam_linear_workspace_bytes(M, N, n_seg, K)
+            ks, rest = divmod(n, M * N * n_seg * 4)
+            assert rest == 0 and (ks == 0 or 2 <= ks <= min(32, K // 64)), (M, N, n_seg, K, n)
+    assert h.wam_linear_workspace_bytes(32, 3072, 1, 14336) == 10 * 32 * 3072 * 4
+    assert h.wam_linear_workspace_bytes(224, 3072, 1, 14336) == 5 * 224 * 3072 * 4
+    assert h.wam_linear_workspace_bytes(224, 14336, 1, 3072) == 0

@@ -1,0 +1,228 @@
+// GEMMs whose 256x256 tiles would leave most of the chip idle: few rows (the
+// action tokens of a policy step, a text context) or few columns.  The plan
+// picks a tile and a number of k ranges so that one round of workgroups
+// covers the CUs; with several ranges the tiles write fp32 partial sums and a
+// reduce pass adds them in range order and applies the epilogue, alone or
+// together with the row pass that follows the projection in the block
+// (RMSNorm + RoPE, or the residual stream and its LayerNorm).
+#include <string.h>
+#include "gemm_tile.h"
+
+namespace wam {
+
+// ------------------------------------------------------------------- tiles
+// What bounds them: a CU keeps about 32 KB of loads in flight, so it takes
+// operands in at 50-60 GB/s while the weights come from HBM, whatever the
+// tile or the way to LDS (224 x 14336 x 3072 on 128x128 tiles: 34 us staged
+// through LDS by direct loads or through registers, 3 or 5 stages).  Fewer
+// operand bytes per output (a larger tile) and more CUs at work are what
+// helps; k ranges trade the second against partial-sum traffic.
+using Small32 = GemmCfg<32, 128, 64, 1, 4, 3, 2>;
+using Small64 = GemmCfg<64, 128, 64, 1, 4, 5>;
+using Small128 = GemmCfg<128, 128, 64, 2, 4, 5, 1, 2>;
+using Small192 = GemmCfg<192, 128, 64, 2, 4, 3, 1, 2>;
+using Small256 = GemmCfg<256, 128, 64, 4, 2, 3, 1, 2>;
+using SmallN256 = GemmCfg<128, 256, 64, 2, 4, 3, 1, 2>;
+// fp8 e4m3 weights (64-byte LDS rows widened at the fragment read)
+using Small64f8 = GemmCfg<64, 128, 64, 1, 4, 5, 1, 0, 1>;
+using Small128f8 = GemmCfg<128, 128, 64, 2, 4, 5, 1, 0, 1>;
+using Small256f8 = GemmCfg<256, 128, 64, 4, 2, 3, 1, 0, 1>;
+
+// Cost model, in us: kLaunch + rounds * (round + steps * step), rounds being
+// dispatch rounds of one workgroup per CU and steps the 64-deep k-steps of
+// one range; at least the weights' time from HBM; and for several ranges the
+// reduce pass, kReduce + kPerMB per MB of partial sums (written and read).
+// Fitted to 34 shapes (96 to 2325 rows, K 1536 to 14336, N 1536 to 14336, 1
+// to 32 ranges, weights cold): 6% rms, and the plan it picks is within 3% of
+// the fastest measured one but for 400 x 3072 x 14336 (8%) and 224 x 9216 x
+// 3072 (13%).  Against 128x128 or 256x128 tiles over the whole k:
+//   32 x 3072 x 14336 107 -> 22 us     780 x 3072 x 14336 114 -> 80
+//   224 x 3072 x 3072  30 -> 18        1024 x 9216 x 3072 104 -> 60
+//   224 x 3072 x 14336 125 -> 37       1560 x 3072 x 14336 227 -> 122
+//   1024 x 1536 x 8960  82 -> 40       2325 x 3072 x 14336 218 -> 182
+struct TileCost {
+  int bm, bn;
+  double round, step;
+};
+constexpr TileCost kTiles[] = {
+    {32, 128, 0.3, 0.47},  {64, 128, 1.9, 0.42},  {128, 128, 3.0, 0.49},  {192, 128, 2.2, 0.64},
+    {256, 128, 2.7, 0.81}, {128, 256, 3.1, 0.82}, {224, 256, 4.7, 1.05},  {256, 256, 4.4, 1.21},
+};
+constexpr int kTile32 = 0, kTile192 = 3, kTileN256 = 5, kTileW224 = 6, kTileCount = 8;
+constexpr double kLaunch = 2.6, kReduce = 4.1, kPerMB = 0.28, kHbmBytesPerUs = 6.6e6;
+constexpr int kMaxRanges = 32;
+
+SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_bytes) {
+  const int cus = device_cu_count(), nk = K / 64;
+  const double hbm = (double)seg_n * n_seg * K * wb / kHbmBytesPerUs;
+  SplitPlan best{0, 1};
+  double best_cost = 1e30;
+  for (int c = 0; c < kTileCount; ++c) {
+    const TileCost& t = kTiles[c];
+    const bool w4 = c >= kTileW224;
+    // 256-column tiles hold whole tiles of one segment; the fp8-weight small
+    // tiles are 128 columns wide
+    if ((w4 && seg_n % 256 != 0) || (n_seg > 1 && seg_n % t.bn != 0)) continue;
+    // fp8 weights: 64, 128, 224 and 256 rows, and 256 x 128 (a 32-row stage
+    // would not hold a 32-row slab of the fp32 epilogue)
+    if (wb == 1 && (c == kTile32 || c == kTile192 || c == kTileN256)) continue;
+    // a shorter tile holds all rows
+    if (c > (wb == 1 ? 1 : 0) && kTiles[c - 1].bm >= M && kTiles[c - 1].bn == t.bn) continue;
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((seg_n + t.bn - 1) / t.bn) * n_seg;
+    // one range, or as many as fill one or two rounds
+    const int64_t cand[3] = {1, cus / tiles, 2 * cus / tiles};
+    for (int64_t ks : cand) {
+      if (ks > kMaxRanges) ks = kMaxRanges;
+      if (ks > nk) ks = nk;
+      if (ks < 1) continue;
+      const int64_t rounds = (tiles * ks + cus - 1) / cus, steps = (nk + ks - 1) / ks;
+      const int64_t bytes = ks > 1 ? ks * (int64_t)M * seg_n * n_seg * 4 : 0;
+      if (bytes > ws_bytes) continue;
+      double cost = (double)rounds * (t.round + (double)steps * t.step);
+      cost = kLaunch + (cost > hbm ? cost : hbm);
+      if (ks > 1) cost += kReduce + kPerMB * 1e-6 * (double)bytes;
+      if (cost < best_cost - 1e-9) best_cost = cost, best = SplitPlan{c, (int)ks};
+    }
+  }
+  return best;
+}
+
+int64_t split_plan_bytes(const SplitPlan& g, int M, int seg_n, int n_seg) {
+  return g.ks > 1 ? g.ks * (int64_t)M * seg_n * n_seg * 4 : 0;
+}
+
+template <class C>
+static int launch_small(LinearParams& p, hipStream_t s) {
+  p.n_tiles_per_seg = (p.seg_n + C::BN - 1) / C::BN;
+  p.m_tiles = (p.M + C::BM - 1) / C::BM;
+  p.n_tiles = p.n_tiles_per_seg * p.n_seg_count;
+  p.part_ld = p.seg_n * p.n_seg_count;
+  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles * p.k_split)), block(C::kThreads);
+  if (p.k_split > 1) {
+    hipLaunchKernelGGL((gemm_bf16_kernel<C, kEpiPartial>), grid, block, 0, s, p);
+  } else {
+    switch (p.epi) {
+      case WAM_EPI_BIAS:
+        hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS>), grid, block, 0, s, p);
+        break;
+      case WAM_EPI_BIAS_GELU:
+        hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS_GELU>), grid, block, 0, s, p);
+        break;
+      case WAM_EPI_BIAS_GATE_RES:
+        if (p.res_f32) hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS_GATE_RES, 1>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS_GATE_RES, 0>), grid, block, 0, s, p);
+        break;
+      default:
+        if (p.res_f32) hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS_RES, 1>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((gemm_bf16_kernel<C, WAM_EPI_BIAS_RES, 0>), grid, block, 0, s, p);
+        break;
+    }
+  }
+  WAM_LAUNCHED("gemm_bf16_kernel");
+  return WAM_OK;
+}
+
+// The tiles of a plan: with several ranges only the partial sums are written.
+int split_tiles(LinearParams& p, const SplitPlan& g, int wb, hipStream_t s) {
+  p.k_split = g.ks;
+  WAM_REQUIRE(g.ks == 1 || (p.part && g.ks <= p.K / 64), "wam_linear: bad split-K launch");
+  if (g.tile >= kTileW224) return w4_tiles(p, kTiles[g.tile].bm, wb, s);
+  if (wb == 1) {
+    switch (g.tile) {
+      case 1: return launch_small<Small64f8>(p, s);
+      case 2: return launch_small<Small128f8>(p, s);
+      default: return launch_small<Small256f8>(p, s);
+    }
+  }
+  switch (g.tile) {
+    case 0: return launch_small<Small32>(p, s);
+    case 1: return launch_small<Small64>(p, s);
+    case 2: return launch_small<Small128>(p, s);
+    case kTile192: return launch_small<Small192>(p, s);
+    case kTileN256: return launch_small<SmallN256>(p, s);
+    default: return launch_small<Small256>(p, s);
+  }
+}
+
+// ------------------------------------------------------------------ reduce
+// Sum of the k_split partial ranges at element offset `at` of a plane, in
+// range order.
+__device__ inline f32x4 sum_ranges(const float* part, int ks, int64_t plane, int64_t at) {
+  f32x4 v = *reinterpret_cast<const f32x4*>(part + at);
+#pragma unroll 8
+  for (int r = 1; r < ks; ++r) v += *reinterpret_cast<const f32x4*>(part + r * plane + at);
+  return v;
+}
+
+__device__ inline void widen4_bf16(u32x2 t, float out[4]) {
+  out[0] = __uint_as_float(t[0] << 16);
+  out[1] = __uint_as_float(t[0] & 0xffff0000u);
+  out[2] = __uint_as_float(t[1] << 16);
+  out[3] = __uint_as_float(t[1] & 0xffff0000u);
+}
+
+// 4 consecutive values of a bf16 or fp32 vector in two unconditional 8-byte
+// loads (for bf16 the second repeats the first), so that none sits in a
+// branch; widen4 makes fp32 values of them.
+struct Raw4 {
+  u32x2 a, b;
+};
+__device__ inline Raw4 ld4_raw(const void* p, bool f32, int64_t off) {
+  const char* base = static_cast<const char*>(p) + off * (f32 ? 4 : 2);
+  return Raw4{*reinterpret_cast<const u32x2*>(base), *reinterpret_cast<const u32x2*>(base + (f32 ? 8 : 0))};
+}
+__device__ inline void widen4(const Raw4& r, bool f32, float out[4]) {
+  float h[4];
+  widen4_bf16(r.a, h);
+  out[0] = f32 ? __uint_as_float(r.a[0]) : h[0];
+  out[1] = f32 ? __uint_as_float(r.a[1]) : h[1];
+  out[2] = f32 ? __uint_as_float(r.b[0]) : h[2];
+  out[3] = f32 ? __uint_as_float(r.b[1]) : h[3];
+}
+
+// The launch's epilogue over the partial sums, one thread per 4 consecutive
+// outputs of one segment.  W1: fp8 weights (per-column scales).
+template <int EPI, bool W1>
+__global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
+  const int q4 = p.part_ld / 4;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)p.M * q4) return;
+  const int m = (int)(i / q4), c = (int)(i - (int64_t)m * q4) * 4;
+  const int seg = c >= p.seg_n ? (c >= 2 * p.seg_n ? 2 : 1) : 0, n = c - seg * p.seg_n;
+  const bf16* bias = seg == 0 ? p.bias[0] : (seg == 1 ? p.bias[1] : p.bias[2]);
+  void* out = seg == 0 ? p.out[0] : (seg == 1 ? p.out[1] : p.out[2]);
+  float bv[4] = {0.f, 0.f, 0.f, 0.f}, wsc[4] = {1.f, 1.f, 1.f, 1.f}, rv[4] = {0.f, 0.f, 0.f, 0.f};
+  const u32x2 braw = *reinterpret_cast<const u32x2*>(bias ? static_cast<const void*>(bias + n) : p.part);
+  if constexpr (W1) {
+    const float* ws = seg == 0 ? p.wscale[0] : (seg == 1 ? p.wscale[1] : p.wscale[2]);
+    const float4 t = *reinterpret_cast<const float4*>(ws + n);
+    wsc[0] = t.x; wsc[1] = t.y; wsc[2] = t.z; wsc[3] = t.w;
+  }
+  constexpr bool RES = EPI == WAM_EPI_BIAS_GATE_RES || EPI == WAM_EPI_BIAS_RES;
+  Raw4 rraw{};
+  if constexpr (RES) rraw = ld4_raw(p.res, p.res_f32 != 0, (int64_t)m * p.ldr + n);
+  const f32x4 v = sum_ranges(p.part, p.k_split, (int64_t)p.M * p.part_ld, (int64_t)m * p.part_ld + c);
+  if (bias) widen4_bf16(braw, bv);
+  if constexpr (RES) widen4(rraw, p.res_f32 != 0, rv);
+  const float no_gate[4] = {0.f, 0.f, 0.f, 0.f};
+  epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v, bv, wsc, no_gate, false, rv);
+}
+
+int split_reduce(const LinearParams& p, int wb, hipStream_t s) {
+  const dim3 grid((unsigned)(((int64_t)p.M * (p.part_ld / 4) + 255) / 256)), block(256);
+  const bool w1 = wb == 1;
+#define WAM_REDUCE(E)                                                                             \
+  if (w1) hipLaunchKernelGGL((split_reduce_kernel<E, true>), grid, block, 0, s, p);               \
+  else hipLaunchKernelGGL((split_reduce_kernel<E, false>), grid, block, 0, s, p)
+  switch (p.epi) {
+    case WAM_EPI_BIAS: WAM_REDUCE(WAM_EPI_BIAS); break;
+    case WAM_EPI_BIAS_GELU: WAM_REDUCE(WAM_EPI_BIAS_GELU); break;
+    case WAM_EPI_BIAS_GATE_RES: WAM_REDUCE(WAM_EPI_BIAS_GATE_RES); break;
+    default: WAM_REDUCE(WAM_EPI_BIAS_RES); break;
+  }
+#undef WAM_REDUCE
+  WAM_LAUNCHED("split_reduce_kernel");
+  return WAM_OK;
+}
+
+}  // namespace wam
