@@ -1,0 +1,154 @@
+"""Attention with few queries per key source (attention_few.hip): 32, 64 and
+128 queries per workgroup, whole and in key ranges, grouped batch rows, key
+sources of every shape, against an fp32 softmax."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle.metrics import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(shape, dev, seed, std=1.0):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    return (torch.randn(shape, generator=g, device=dev) * std).to(torch.bfloat16)
+
+
+def _ref(q, k, v, ks):
+    """fp32 attention of q [B, Mq, H, hd] over per-row key lists."""
+    out = []
+    for b in range(q.shape[0]):
+        s = torch.einsum("qhd,khd->hqk", q[b].float(), ks[b][0].float()) / 128 ** 0.5
+        out.append(torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), ks[b][1].float()))
+    return torch.stack(out)
+
+
+def _pool(dev, Bp, P, H, valid, seed):
+    slots = torch.zeros(P, dtype=torch.int32, device=dev)
+    slots[:valid.numel()] = valid.int()
+    run = int(valid[0]) if valid.numel() and int(valid[-1] - valid[0]) + 1 == valid.numel() else -1
+    return dict(pool_k=_randn((Bp, P, H, 128), dev, seed), pool_v=_randn((Bp, P, H, 128), dev, seed + 1), slots=slots,
+                n_hist=torch.tensor([valid.numel()], dtype=torch.int32, device=dev),
+                hist_base=torch.tensor([run], dtype=torch.int32, device=dev))
+
+
+# Own keys: one key, a tile, one more; 33 queries (two waves' worth of rows in
+# one workgroup size up), 65 to 129 queries, a last partial workgroup, few
+# queries over many keys (ranges and the merge).
+@pytest.mark.parametrize("B,Mq,Mk,H", [(1, 1, 1, 1), (2, 16, 32, 24), (2, 31, 33, 24), (1, 33, 500, 24), (3, 65, 129, 12),
+                                       (1, 129, 512, 24), (2, 200, 96, 12), (1, 780, 512, 24), (1, 1024, 1024, 12),
+                                       (1, 16, 6017, 24), (1, 48, 3001, 24), (1, 500, 2000, 12)])
+def test_own_keys(dev, B, Mq, Mk, H):
+    from wam_ops import ops
+    q, k, v = _randn((B, Mq, H, 128), dev, 1, 2.0), _randn((B, Mk, H, 128), dev, 2), _randn((B, Mk, H, 128), dev, 3)
+    ref = _ref(q, k, v, list(zip(k, v)))
+    assert_close(ops.attention(q, k, v), ref, 2e-2, 0.9999, f"own keys {B}x{Mq}x{Mk}x{H}")
+
+
+# One own row for every batch row (a shared text context): the batch rows run
+# as one list of queries; strided rows of a packed projection do not.
+@pytest.mark.parametrize("B,Mq,Mk", [(14, 16, 512), (2, 128, 77), (7, 5, 40)])
+def test_shared_own_row(dev, B, Mq, Mk):
+    from wam_ops import ops
+    H = 24
+    packed = _randn((B, Mq, 3, H, 128), dev, 1, 2.0)
+    k, v = _randn((1, Mk, H, 128), dev, 2), _randn((1, Mk, H, 128), dev, 3)
+    for q in (packed[:, :, 0], packed[:, :, 0].contiguous(), packed[:, :, 0].contiguous().transpose(0, 1).contiguous()
+              .transpose(0, 1)):
+        ref = _ref(q, k, v, [(k[0], v[0])] * B)
+        assert_close(ops.attention(q, k, v), ref, 2e-2, 0.9999, f"shared own row {B}x{Mq}x{Mk}")
+
+
+# A pool: consecutive slots, a gap (listed slots), no valid slot; candidates
+# of one and two pool rows in and out of order (groups of two batch rows of
+# one, of two and of three rows of different pool rows).
+@pytest.mark.parametrize("B,Mq,n,gap,rows", [
+    (2, 16, 288, 0, None), (2, 16, 290, 7, None), (2, 100, 1000, 50, None), (2, 16, 0, 0, None),
+    (14, 16, 1152, 0, [0] * 7 + [1] * 7), (14, 16, 720, 3, [0, 1] * 7), (14, 16, 100, 0, [1] * 14),
+    (6, 9, 65, 1, [0, 0, 0, 0, 1, 1]), (4, 8, 33, 0, [1, 0, 0, 0]), (1, 20, 6000, 0, [1]), (7, 48, 900, 0, [0] * 7),
+    (2, 16, 5000, 11, [0, 0])])
+def test_pool(dev, B, Mq, n, gap, rows):
+    from wam_ops import ops
+    H, Bp = 24, (B if rows is None else 2)
+    q, k, v = _randn((B, Mq, H, 128), dev, 1, 2.0), _randn((B, Mq, H, 128), dev, 2), _randn((B, Mq, H, 128), dev, 3)
+    valid = torch.arange(n, device=dev)
+    valid[n // 2:] += gap
+    kw = _pool(dev, Bp, n + gap + 5, H, valid + 3, 4)
+    if rows is not None:
+        kw["pool_rows"] = torch.tensor(rows, dtype=torch.int64, device=dev)
+    at = rows if rows is not None else range(B)
+    src = [(torch.cat([kw["pool_k"][r][valid + 3], k[b]]), torch.cat([kw["pool_v"][r][valid + 3], v[b]]))
+           for b, r in enumerate(at)]
+    # what lies past the valid slots must not reach the result
+    dead = torch.ones(n + gap + 5, dtype=torch.bool, device=dev)
+    dead[valid + 3] = False
+    kw["pool_k"][:, dead] = float("nan")
+    kw["pool_v"][:, dead] = float("inf")
+    assert_close(ops.attention(q, k, v, **kw), _ref(q, k, v, src), 2e-2, 0.9999, f"pool {B}x{Mq} over {n}")
+
+
+def test_own_row_map_and_query_rms(dev):
+    """kv_rows, and q_ssq's per-query factor (rows of the folded batch too)."""
+    from wam_ops import ops
+    B, Mq, Mk, H = 6, 12, 70, 24
+    q, k, v = _randn((B, Mq, H, 128), dev, 1, 2.0), _randn((2, Mk, H, 128), dev, 2), _randn((2, Mk, H, 128), dev, 3)
+    rows = torch.tensor([0, 1, 1, 0, 0, 1], device=dev)
+    src = [(k[r], v[r]) for r in rows.tolist()]
+    assert_close(ops.attention(q, k, v, kv_rows=rows), _ref(q, k, v, src), 2e-2, 0.9999, "own row map")
+    ssq = (torch.rand(B * Mq, 12, device=dev) + 0.5) * 256
+    f = torch.rsqrt(ssq.sum(1) / (H * 128) + 1e-6).view(B, Mq, 1, 1)
+    ref = _ref(q.float() * f, k, v, [(k[0], v[0])] * B)
+    assert_close(ops.attention(q, k[:1], v[:1], q_ssq=ssq), ref, 2e-2, 0.9999, "query RMS factor")
+
+
+@pytest.mark.parametrize("B,Mq,Mk", [(1, 16, 6000), (1, 48, 3000)])
+def test_workspace_sizes(dev, B, Mq, Mk):
+    """No workspace, one short of the plan's, the plan's, and the entry point
+    without allocation: the same call, in as many ranges as fit."""
+    from wam_ops import _lib
+    H = 24
+    q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, Mk, H, 128), dev, 2), _randn((B, Mk, H, 128), dev, 3)
+    ref = _ref(q, k, v, list(zip(k, v)))
+    h = _lib.lib()
+    need = h.wam_attention_workspace_bytes(B, Mq, H, Mk)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    outs = []
+    for nbytes in (0, need - 1, need, None):
+        o = torch.zeros_like(q)
+        a = _lib.AttentionArgs()
+        a.q, a.q_bstride, a.q_rstride = q.data_ptr(), q.stride(0), q.stride(1)
+        a.o, a.o_bstride, a.o_rstride = o.data_ptr(), o.stride(0), o.stride(1)
+        a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch, a.scale, a.max_keys = B, Mq, H, 128, Mk, B, 128 ** -0.5, Mk
+        a.k, a.v, a.kv_bstride, a.kv_rstride = k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1)
+        if nbytes:
+            a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
+        f = h.wam_attention if nbytes is not None else h.wam_attention_noalloc
+        _lib.check(f(ctypes.byref(a), None), "wam_attention")
+        torch.cuda.synchronize()
+        assert_close(o, ref, 2e-2, 0.9999, f"workspace of {nbytes} bytes")
+        outs.append(o)
+    assert torch.equal(outs[2], outs[3])
+
+
+def test_candidates_are_isolated(dev):
+    """A candidate whose own rows hold infinities and NaN leaves the others,
+    its neighbour in the same workgroup too, as they were."""
+    from wam_ops import ops
+    B, Mq, H, n = 14, 16, 24, 200
+    q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, Mq, H, 128), dev, 2), _randn((B, Mq, H, 128), dev, 3)
+    kw = _pool(dev, 2, n, H, torch.arange(n, device=dev), 4)
+    kw["pool_rows"] = torch.tensor([0] * 7 + [1] * 7, device=dev)
+    clean = ops.attention(q, k, v, **kw)
+    v[4], k[4, 3], v[9, 0] = float("inf"), float("nan"), float("nan")
+    out = ops.attention(q, k, v, **kw)
+    keep = [b for b in range(B) if b not in (4, 9)]
+    assert torch.equal(out[keep], clean[keep])
+    assert not bool(torch.isfinite(out[[4, 9]].float()).any())
+    # the other branch's history (rows 6 and 7 share a workgroup)
+    kw["pool_v"][1] = float("inf")
+    out = ops.attention(q, k, v, **kw)
+    assert torch.equal(out[[0, 6]], clean[[0, 6]])

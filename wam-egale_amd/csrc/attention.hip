@@ -22,39 +22,9 @@
 // place through the slot list.
 #include <algorithm>
 #include <mutex>
-#include "wam_common.h"
+#include "attention_common.h"
 
 namespace wam {
-
-constexpr int kAttnHD = 128;
-constexpr int kAttnKT = 64;                          // keys per LDS stage
-constexpr int kAttnTile = kAttnKT * kAttnHD * 2;     // 16 KB per K or V tile
-constexpr int kAttnStage = 2 * kAttnTile;            // K tile + V tile
-constexpr int kAttnStages = 3;
-
-// LDS layouts (64 banks x 4 bytes; 256-byte rows = one bank line).
-// K [64 keys][128 d]: an S^T operand fetch reads 16 consecutive keys at one
-// 16-byte chunk per cycle, so chunk XOR (key mod 16).
-__device__ inline int k_off(int key, int c) { return key * 256 + ((c ^ (key & 15)) << 4); }
-// V [64 keys][128 d] in natural layout: a transposed read fetches 4
-// consecutive keys x 64 bytes per 32 lanes, so the 64-byte segment XOR
-// (key mod 4).
-__device__ inline int v_off(int key, int c) { return key * 256 + ((c ^ ((key & 3) << 2)) << 4); }
-
-__device__ inline int clamp_row(int r, int n) { return r < 0 ? 0 : (r >= n ? n - 1 : r); }
-
-// Per-query RMS factor of queries written by wam_linear's norm epilogue:
-// rsqrt(sum of the row's q_ssq_n partial sums of squares / q_norm_dim + eps)
-// for query row b * Mq + qi (clamped into range).  The RMSNorm across heads
-// is model.py:609-612; the rotation after it is linear and commutes.  The
-// pipelined kernel stages the partial sums through LDS instead (see there).
-constexpr int kQssqMax = 16;
-__device__ inline float q_rms_factor(const wam_attention_args& a, int b, int qi) {
-  const float* p = a.q_ssq + ((int64_t)b * a.Mq + min(qi, a.Mq - 1)) * a.q_ssq_n;
-  float s = 0.f;
-  for (int t = 0; t < a.q_ssq_n; ++t) s += p[t];
-  return rsqrtf(s / (float)a.q_norm_dim + a.q_eps);
-}
 
 // Workgroup: W waves x 32 queries of one (batch row, head).  Wave w owns
 // queries q0 + 32 w .. +32 and keeps its Q fragments in registers.
@@ -1115,10 +1085,52 @@ static int query_tile(const wam_attention_args* a, int64_t keys) {
   return sp_eligible(a) && a->n_hist_dev == nullptr ? sp_query_tile(a->B, a->Mq, a->H, keys) : 256;
 }
 
+// Time of the 256-query kernels for the call, in us, as measured on 40 shapes
+// of 4 to 1500 queries (mostly within 20%): the launches and the merge, and
+// the key tiles that one CU runs one after another, cheaper with fewer live
+// queries and in the pipelined kernel, there cheaper without pool keys.
+static double plan_us(const wam_attention_args* a, int64_t keys, int64_t ws_bytes) {
+  const AttnPlan p = attention_plan(a->B, a->Mq, a->H, keys, ws_bytes, 256);
+  const int64_t cus = device_cu_count(), pieces = (int64_t)p.n_tail * p.n_split;
+  const double kt = (double)((keys + kAttnKT - 1) / kAttnKT), live = std::min(a->Mq, 256) / 256.0;
+  const double tiles = kt * ((double)((p.n_full + cus - 1) / cus) + (double)((pieces + cus - 1) / cus) / p.n_split);
+  const double tile = sp_eligible(a) ? (a->n_hist_dev ? 1.2 : 0.7) : 1.43;
+  return (p.n_split > 1 ? 11.0 + 4.0 * live : 6.0) + tiles * (tile + 1.3 * live);
+}
+
+// Whether the few-query kernel takes the call: row offsets within its 32-bit
+// buffer offsets, and a plan that is predicted to be faster.  `call` is the
+// call it runs: when every batch row attends to the same own keys and nothing
+// else, and the rows of q and o follow one another, the batch rows are one
+// run of B * Mq queries (14 x 16 queries over one text context: whole waves).
+static bool takes_few(const wam_attention_args* a, int64_t ws_bytes, wam_attention_args* call, FewPlan* few) {
+  const int64_t keys = a->max_keys > 0 ? a->max_keys : a->Mk;
+  if (((int64_t)a->Mk + 64) * a->kv_rstride * 2 >= (int64_t)INT32_MAX) return false;
+  if (a->n_hist_dev && (a->pool_bstride < a->pool_rstride || a->pool_bstride * 2 >= (int64_t)INT32_MAX)) return false;
+  *call = *a;
+  if (a->B > 1 && !a->n_hist_dev && !a->kv_rows && a->kv_batch == 1 && a->q_bstride == a->Mq * a->q_rstride &&
+      a->o_bstride == a->Mq * a->o_rstride && (int64_t)a->B * a->Mq < (1 << 26)) {
+    call->Mq = a->B * a->Mq;
+    call->B = 1;
+  }
+  const int sharing = a->n_hist_dev && a->pool_rows ? std::max(1, a->B / a->pool_batch) : 1;
+  *few = attention_few_plan(call->B, call->Mq, call->H, keys, sharing, ws_bytes);
+  return few->qw != 0 && few->cost < 0.95 * plan_us(a, keys, ws_bytes);
+}
+
 int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys) {
-  // enough for either query tile (the call's strides, unknown here, decide)
-  return std::max(plan_bytes(attention_plan(B, Mq, H, max_keys, INT64_MAX, 256)),
-                  plan_bytes(attention_plan(B, Mq, H, max_keys, INT64_MAX, sp_query_tile(B, Mq, H, max_keys))));
+  // enough for either query tile, and for the few-query kernel with any
+  // grouping of batch rows (the call's strides and row maps, unknown here,
+  // decide)
+  int64_t most = std::max(plan_bytes(attention_plan(B, Mq, H, max_keys, INT64_MAX, 256)),
+                          plan_bytes(attention_plan(B, Mq, H, max_keys, INT64_MAX, sp_query_tile(B, Mq, H, max_keys))));
+  auto few = [&](int b, int m, int sharing) {
+    const FewPlan p = attention_few_plan(b, m, H, max_keys, sharing, INT64_MAX);
+    if (p.qw) most = std::max(most, attention_few_bytes(p, b, m, H));
+  };
+  for (int sharing = 1; sharing <= 8; ++sharing) few(B, Mq, sharing);
+  if (B > 1 && (int64_t)B * Mq < (1 << 26)) few(1, B * Mq, 1);
+  return most;
 }
 
 int attention(const wam_attention_args* a, hipStream_t s) {
@@ -1149,6 +1161,10 @@ int attention(const wam_attention_args* a, hipStream_t s) {
               "wam_attention: q_ssq needs 1..%d partials per row and q_norm_dim >= 1 (got %d, %d)", kQssqMax,
               a->q_ssq_n, a->q_norm_dim);
   if (a->Mq == 0) return WAM_OK;
+  wam_attention_args call;
+  FewPlan few;
+  if (takes_few(a, a->workspace ? a->workspace_bytes : 0, &call, &few))
+    return attention_few(&call, few, static_cast<float*>(a->workspace), s);
   // 8 or 7 waves (256 or 224 queries) per workgroup, with the last dispatch
   // round split by key ranges when the plan says so and the caller gave a
   // workspace for the partial results; small grids use 4-wave workgroups.
@@ -1239,12 +1255,18 @@ int attention_noalloc(const wam_attention_args* a, hipStream_t s) {
   // whose partial results exceed the scratch are refused, not re-planned, so
   // that both entry points compute the same thing.
   const int64_t keys = a->max_keys > 0 ? a->max_keys : a->Mk;
-  const int64_t need =
+  int64_t need =
       a->Mq > 0 ? plan_bytes(attention_plan(a->B, a->Mq, a->H, keys, INT64_MAX, query_tile(a, keys))) : 0;
   WAM_REQUIRE(need <= kNoAllocScratchBytes,
               "wam_attention_noalloc: this shape's key-range split needs %lld bytes of scratch, more than "
               "the %lld-byte maximum; call wam_attention with a workspace instead",
               (long long)need, (long long)kNoAllocScratchBytes);
+  // (the few-query kernel's ranges, at most 256 partial tiles of 128 queries,
+  // always fit)
+  wam_attention_args call;
+  FewPlan few;
+  if (a->Mq > 0 && takes_few(a, kNoAllocScratchBytes, &call, &few))
+    need = attention_few_bytes(few, call.B, call.Mq, call.H);
   wam_attention_args b = *a;
   if (need > 0) {
     void* p = nullptr;
