@@ -24,7 +24,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <vector>
-#include "wam_common.h"
+#include "gemm_tile.h"
 
 namespace wam {
 
@@ -107,6 +107,8 @@ static Layout layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
   // One region: the kernels that use it run one after another on the stream.
   const int64_t need[] = {attention_workspace_bytes(B, M, D / 128, (int64_t)M + (pool > 0 ? pool : 0)),
                           attention_workspace_bytes(B, M, D / 128, Lc),
+                          linear_workspace_bytes((int)R, D, 3, D),   // QKV
+                          linear_workspace_bytes(Bc * Lc, D, 2, D),  // cross K/V
                           linear_workspace_bytes((int)R, D, 1, D),   // self_out, cross_q, cross_out
                           linear_workspace_bytes((int)R, F, 1, D),   // FFN1
                           linear_workspace_bytes((int)R, D, 1, F)};  // FFN2
@@ -185,11 +187,12 @@ static void gemm_args(wam_linear_args& g, const void* a, int64_t lda, int M, int
 
 // Cross K/V of the context rows: k = RMS(ctx Wk^T + bk) g, v = ctx Wv^T + bv.
 static int context_kv(const wam_block_weights* W, const void* ctx, int rows, void* k, void* v,
-                      hipStream_t s, void* k_linear_debug = nullptr) {
+                      hipStream_t s, void* k_linear_debug = nullptr, void* ws = nullptr, int64_t ws_bytes = 0) {
   const int D = W->dim;
   wam_linear_args g;
   gemm_args(g, ctx, D, rows, D, D, W->w[15], W->w[16], k, D);
   g.n_seg = 2; g.w[1] = W->w[17]; g.bias[1] = W->w[18]; g.out[1] = v;
+  g.workspace = ws; g.workspace_bytes = ws_bytes;
   WAM_TRY(linear(&g, s));
   if (k_linear_debug)
     WAM_HIP(hipMemcpyAsync(k_linear_debug, k, (size_t)rows * D * 2, hipMemcpyDeviceToDevice, s));
@@ -317,6 +320,10 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
                        dim3(256), 0, s, mod, D, n, static_cast<float*>(dbg(27)));
     WAM_LAUNCHED("modulation_table_kernel");
   }
+  // With few rows a projection runs split over k and leaves its partial sums
+  // to the row pass that follows it.
+  LinearParams sp;
+  bool split = false;
   // 2. Q|K|V projection as one launch into the packed [R, 3D] buffer.
   {
     Scope sc(a->timer, WAM_STAGE_QKV, s);
@@ -326,18 +333,28 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     g.w[1] = W->w[5]; g.bias[1] = W->w[6]; g.out[1] = qkv + D;
     g.w[2] = W->w[7]; g.bias[2] = W->w[8]; g.out[2] = qkv + 2 * D;
     g.workspace = split_ws; g.workspace_bytes = split_bytes;
-    WAM_TRY(linear(&g, s));
+    WAM_TRY(linear_partials(&g, s, &sp, &split));
+    if (!split) WAM_TRY(linear(&g, s));
   }
-  for (int i = 0; i < 2; ++i) {
-    if (dbg(15 + i))
-      WAM_HIP(hipMemcpy2DAsync(dbg(15 + i), D * 2, qkv + i * D, 3 * D * 2, D * 2, R, hipMemcpyDeviceToDevice, s));
-    if (dbg(17 + i)) {
-      wam_rms_rope_args r{};
-      r.x[0] = qkv + i * D; r.y[0] = dbg(17 + i); r.gamma[0] = W->w[11 + i]; r.eps[0] = W->eps[3 + i];
-      r.ldx = 3 * D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
-      WAM_TRY(rms_rope(&r, s));
+  // Debug copies of the projections before and after their norm: of the
+  // buffer before the norm overwrites it, or by launches of their own after
+  // the row pass that formed q, k and v from partial sums.
+  auto qk_debug = [&]() -> int {
+    for (int i = 0; i < 2; ++i) {
+      void* lin = dbg(15 + i) ? dbg(15 + i) : dbg(17 + i);
+      if (split && lin) WAM_TRY(plain_linear(h, D, D, 3 + 2 * i, -1, lin));
+      else if (dbg(15 + i))
+        WAM_HIP(hipMemcpy2DAsync(dbg(15 + i), D * 2, qkv + i * D, 3 * D * 2, D * 2, R, hipMemcpyDeviceToDevice, s));
+      if (dbg(17 + i)) {
+        wam_rms_rope_args r{};
+        r.x[0] = split ? lin : qkv + i * D; r.y[0] = dbg(17 + i); r.gamma[0] = W->w[11 + i]; r.eps[0] = W->eps[3 + i];
+        r.ldx = split ? D : 3 * D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
+        WAM_TRY(rms_rope(&r, s));
+      }
     }
-  }
+    return WAM_OK;
+  };
+  if (!split) WAM_TRY(qk_debug());
   // 3. q/k RMSNorm across heads + RoPE, in place.
   {
     Scope sc(a->timer, WAM_STAGE_RMS_ROPE, s);
@@ -347,8 +364,9 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     r.ldx = 3 * D; r.ldy = 3 * D; r.n_tensors = 2; r.rows = R; r.D = D;
     r.head_dim = W->head_dim;
     r.freq = a->freq; r.freq_batch = a->freq_batch; r.tokens = M;
-    WAM_TRY(rms_rope(&r, s));
+    WAM_TRY(split ? split_rms_rope(sp, r, s) : rms_rope(&r, s));
   }
+  if (split) WAM_TRY(qk_debug());
   if (a->debug) {
     for (int i = 0; i < 3; ++i)
       if (a->debug[1 + i])
@@ -404,10 +422,10 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     g.epilogue = WAM_EPI_BIAS_GATE_RES; g.res = a->x; g.ldr = D; g.gate = mod; g.gate_index = 2;
     g.out_dtype = WAM_F32;
     g.workspace = split_ws; g.workspace_bytes = split_bytes;
-    WAM_TRY(linear(&g, s));
+    split = false;
+    if (W->w[1]) WAM_TRY(linear_partials(&g, s, &sp, &split));
+    if (!split) WAM_TRY(linear(&g, s));
   }
-  WAM_TRY(copy_debug(a->debug, 5, x1, rowb * 2, s));
-  if (dbg(19)) WAM_TRY(plain_linear(attn, D, D, 9, -1, dbg(19)));
   // 8. norm2 (affine LayerNorm), or without cross_attn_norm the bf16 cast
   //    of the residual stream that the identity norm2 passes through.
   const bf16* n2 = h;
@@ -417,11 +435,13 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       wam_ln_args l{};
       l.x = x1; l.x_dtype = WAM_F32; l.y = h; l.rows = R; l.D = D; l.eps = W->eps[1]; l.affine = 1;
       l.gamma = W->w[1]; l.beta = W->w[2]; l.gb_dtype = W->norm2_dtype;
-      WAM_TRY(ln_modulate(&l, s));
+      WAM_TRY(split ? split_ln(sp, l, s) : ln_modulate(&l, s));
     } else {
       WAM_TRY(cast_f32_bf16(x1, h, (int64_t)R * D, s));
     }
   }
+  WAM_TRY(copy_debug(a->debug, 5, x1, rowb * 2, s));
+  if (dbg(19)) WAM_TRY(plain_linear(attn, D, D, 9, -1, dbg(19)));
   WAM_TRY(copy_debug(a->debug, 6, n2, rowb, s));
   // 9. Cross Q = RMS(n2 Wq2^T + b) g  (into the q third of the qkv buffer).
   bf16* cq = qkv;
@@ -431,13 +451,15 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     gemm_args(g, n2, D, R, D, D, W->w[13], W->w[14], cq, D);
     g.workspace = split_ws; g.workspace_bytes = split_bytes;
     if (qnorm_fused) { g.norm_ssq[0] = qssq; g.norm_gamma[0] = W->w[21]; }
-    WAM_TRY(linear(&g, s));
+    split = false;
+    if (!qnorm_fused) WAM_TRY(linear_partials(&g, s, &sp, &split));
+    if (!split) WAM_TRY(linear(&g, s));
     if (!qnorm_fused) {
-      WAM_TRY(copy_debug(a->debug, 20, cq, rowb, s));
+      if (!split) WAM_TRY(copy_debug(a->debug, 20, cq, rowb, s));
       wam_rms_rope_args r{};
       r.x[0] = cq; r.y[0] = cq; r.gamma[0] = W->w[21]; r.eps[0] = W->eps[5];
       r.ldx = D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
-      WAM_TRY(rms_rope(&r, s));
+      WAM_TRY(split ? split_rms_rope(sp, r, s) : rms_rope(&r, s));
     }
   }
   if (qnorm_fused) {
@@ -453,6 +475,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       WAM_TRY(rms_rope(&r, s));
     }
   } else {
+    if (split && dbg(20)) WAM_TRY(plain_linear(n2, D, D, 13, -1, dbg(20)));
     WAM_TRY(copy_debug(a->debug, 7, cq, rowb, s));
   }
   // 10. Cross K/V: precomputed or from the context.
@@ -461,7 +484,8 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
   const size_t ctxb = (size_t)a->context_batch * a->context_len * D * 2;
   if (!precomputed) {
     Scope sc(a->timer, WAM_STAGE_CROSS_KV, s);
-    WAM_TRY(context_kv(W, a->context, a->context_batch * a->context_len, ws + L.ck, ws + L.cv, s, dbg(21)));
+    WAM_TRY(context_kv(W, a->context, a->context_batch * a->context_len, ws + L.ck, ws + L.cv, s, dbg(21),
+                       split_ws, split_bytes));
     ck = ws + L.ck;
     cv = ws + L.cv;
   }
@@ -492,11 +516,9 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     g.epilogue = WAM_EPI_BIAS_RES; g.res = x1; g.ldr = D; g.res_dtype = WAM_F32;
     g.out_dtype = WAM_F32;
     g.workspace = split_ws; g.workspace_bytes = split_bytes;
-    WAM_TRY(linear(&g, s));
+    WAM_TRY(linear_partials(&g, s, &sp, &split));
+    if (!split) WAM_TRY(linear(&g, s));
   }
-  WAM_TRY(copy_debug(a->debug, 11, x2, rowb * 2, s));
-  if (dbg(22)) WAM_TRY(plain_linear(attn, D, D, 19, -1, dbg(22)));
-  if (dbg(26)) WAM_TRY(plain_ln(x2, WAM_F32, W->eps[2], dbg(26)));
   // 13. LN3 + modulation (c_shift 3, c_scale 4).
   {
     Scope sc(a->timer, WAM_STAGE_LN3, s);
@@ -508,8 +530,11 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       l.y8 = h8; l.y8_scale = h8s;
       if (!dbg(12)) l.y = nullptr;
     }
-    WAM_TRY(ln_modulate(&l, s));
+    WAM_TRY(split ? split_ln(sp, l, s) : ln_modulate(&l, s));
   }
+  WAM_TRY(copy_debug(a->debug, 11, x2, rowb * 2, s));
+  if (dbg(22)) WAM_TRY(plain_linear(attn, D, D, 19, -1, dbg(22)));
+  if (dbg(26)) WAM_TRY(plain_ln(x2, WAM_F32, W->eps[2], dbg(26)));
   WAM_TRY(copy_debug(a->debug, 12, h, rowb, s));
   if (dbg(23)) WAM_TRY(plain_linear(h, D, F, 23, 0, dbg(23)));
   // 14. FFN1 + GELU(tanh).

@@ -991,7 +991,8 @@ bool linear_norm_in_epilogue(int M, int seg_n, int n_seg, int K, int64_t ws_byte
   return gemm_plan(M, seg_n, n_seg, K, cus, ws_bytes).kind == 0;
 }
 
-int linear(const wam_linear_args* a, hipStream_t s) {
+// The contract of a call, and its launch parameters.
+static int linear_setup(const wam_linear_args* a, LinearParams& p) {
   WAM_REQUIRE(a != nullptr, "wam_linear: null args");
   WAM_REQUIRE(a->n_seg >= 1 && a->n_seg <= 3, "wam_linear: n_seg must be 1..3 (got %d)", a->n_seg);
   WAM_REQUIRE(a->M >= 1 && a->K >= 1 && a->seg_n >= 1, "wam_linear: empty shape M=%d K=%d N=%d",
@@ -1036,7 +1037,7 @@ int linear(const wam_linear_args* a, hipStream_t s) {
     WAM_REQUIRE(a->gate.temb_mods != 1 && a->gate_index >= 0 && a->gate_index < 6,
                 "wam_linear: the gate reads a [.., 6, D] temb (index %d)", a->gate_index);
   }
-  LinearParams p{};
+  p = LinearParams{};
   p.a = static_cast<const bf16*>(a->a); p.lda = a->lda; p.M = a->M; p.K = a->K;
   p.seg_n = a->seg_n; p.ldw = a->ldw; p.ldo = a->ldo; p.epi = a->epilogue;
   for (int i = 0; i < 3; ++i) {
@@ -1056,7 +1057,6 @@ int linear(const wam_linear_args* a, hipStream_t s) {
   WAM_REQUIRE(a->workspace_bytes >= 0, "wam_linear: negative workspace_bytes");
   p.k_split = 1;
   p.part = static_cast<float*>(a->workspace);
-  const int64_t ws_bytes = a->workspace ? a->workspace_bytes : 0;
   const bool norm = a->norm_ssq[0] || a->norm_ssq[1] || a->norm_ssq[2];
   if (norm) {
     WAM_REQUIRE(a->epilogue == WAM_EPI_BIAS && !f8 && a->out_dtype == WAM_BF16,
@@ -1080,6 +1080,26 @@ int linear(const wam_linear_args* a, hipStream_t s) {
     }
     p.ssq_ld = (a->seg_n + 255) / 256;
   }
+  return WAM_OK;
+}
+
+int linear_partials(const wam_linear_args* a, hipStream_t s, LinearParams* p, bool* split) {
+  *split = false;
+  WAM_TRY(linear_setup(a, *p));
+  if (a->w_dtype != WAM_BF16 || a->a_dtype != WAM_BF16 || uses_big_tiles(a->M, a->seg_n, a->n_seg)) return WAM_OK;
+  const SplitPlan g = split_plan(a->M, a->seg_n, a->n_seg, a->K, 2, a->workspace ? a->workspace_bytes : 0);
+  if (g.ks == 1) return WAM_OK;
+  *split = true;
+  return split_tiles(*p, g, 2, s);
+}
+
+int linear(const wam_linear_args* a, hipStream_t s) {
+  LinearParams p;
+  WAM_TRY(linear_setup(a, p));
+  const bool f8 = a->w_dtype == WAM_FP8, a8 = a->a_dtype == WAM_FP8, amx = a->a_dtype == WAM_FP8_MX;
+  const bool mxo = a->out_dtype == WAM_FP8_MX;
+  const bool norm = a->norm_ssq[0] || a->norm_ssq[1] || a->norm_ssq[2];
+  const int64_t ws_bytes = a->workspace ? a->workspace_bytes : 0;
   const bool big = uses_big_tiles(a->M, a->seg_n, a->n_seg);
   if (a8 || amx) {
     WAM_REQUIRE(f8 && (amx ? a->a_block_scale != nullptr : a->a_scale != nullptr),

@@ -145,41 +145,6 @@ int split_tiles(LinearParams& p, const SplitPlan& g, int wb, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ reduce
-// Sum of the k_split partial ranges at element offset `at` of a plane, in
-// range order.
-__device__ inline f32x4 sum_ranges(const float* part, int ks, int64_t plane, int64_t at) {
-  f32x4 v = *reinterpret_cast<const f32x4*>(part + at);
-#pragma unroll 8
-  for (int r = 1; r < ks; ++r) v += *reinterpret_cast<const f32x4*>(part + r * plane + at);
-  return v;
-}
-
-__device__ inline void widen4_bf16(u32x2 t, float out[4]) {
-  out[0] = __uint_as_float(t[0] << 16);
-  out[1] = __uint_as_float(t[0] & 0xffff0000u);
-  out[2] = __uint_as_float(t[1] << 16);
-  out[3] = __uint_as_float(t[1] & 0xffff0000u);
-}
-
-// 4 consecutive values of a bf16 or fp32 vector in two unconditional 8-byte
-// loads (for bf16 the second repeats the first), so that none sits in a
-// branch; widen4 makes fp32 values of them.
-struct Raw4 {
-  u32x2 a, b;
-};
-__device__ inline Raw4 ld4_raw(const void* p, bool f32, int64_t off) {
-  const char* base = static_cast<const char*>(p) + off * (f32 ? 4 : 2);
-  return Raw4{*reinterpret_cast<const u32x2*>(base), *reinterpret_cast<const u32x2*>(base + (f32 ? 8 : 0))};
-}
-__device__ inline void widen4(const Raw4& r, bool f32, float out[4]) {
-  float h[4];
-  widen4_bf16(r.a, h);
-  out[0] = f32 ? __uint_as_float(r.a[0]) : h[0];
-  out[1] = f32 ? __uint_as_float(r.a[1]) : h[1];
-  out[2] = f32 ? __uint_as_float(r.b[0]) : h[2];
-  out[3] = f32 ? __uint_as_float(r.b[1]) : h[3];
-}
-
 // The launch's epilogue over the partial sums, one thread per 4 consecutive
 // outputs of one segment.  W1: fp8 weights (per-column scales).
 template <int EPI, bool W1>

@@ -16,6 +16,8 @@
 
 namespace wam {
 
+int row_ln(const wam_ln_args& l, hipStream_t s);
+
 // ------------------------------------------------------------- LayerNorm
 // One wave per row, 8 rows per workgroup.  The per-column vectors the rows
 // multiply and add (1 + scale and shift of the modulation, or gamma and beta)
@@ -252,6 +254,20 @@ static void launch_ln(const wam_ln_args* a, hipStream_t s) {
   else hipLaunchKernelGGL((ln_modulate_kernel<8, XF32, Q8>), grid, block, 0, s, *a);
 }
 
+// Few rows take a workgroup each (split_rows.hip): 8 rows of one workgroup
+// leave most CUs without work (back to back, 3072 columns: 224 rows 5.1-5.3
+// -> 4.0 us, 400 rows 5.3-5.7 -> 4.9-5.2, 780 rows 6.4 -> 7.9, so not there;
+// 1536 columns: 3.8 -> 3.3 at 224 rows, even at 400).  With coefficients per
+// token there is nothing for 8 rows to share, and the row's four coefficient
+// vectors come in together there instead of chunk by chunk (fp32 input: 32
+// rows 7.3 -> 3.7 us, 2325 rows 20.9 -> 17.5, 4680 rows 35.2 -> 30.7; 1536
+// columns 1024 rows 6.3 -> 6.0, 4680 rows 17.8 -> 20.1).
+static bool takes_row_ln(const wam_ln_args* a) {
+  if (a->rows <= 400) return true;
+  const bool per_token = !a->affine && a->mod.temb_len == a->mod.tokens && a->mod.tokens > 1;
+  return per_token && (a->D > 2048 || a->rows <= 1024);
+}
+
 int ln_modulate(const wam_ln_args* a, hipStream_t s) {
   WAM_REQUIRE(a != nullptr, "wam_ln_modulate: null args");
   WAM_REQUIRE(a->rows >= 0 && a->D > 0 && a->D % 8 == 0 && a->D <= 4096,
@@ -268,6 +284,7 @@ int ln_modulate(const wam_ln_args* a, hipStream_t s) {
                 a->shift_index);
   }
   if (a->rows == 0) return WAM_OK;
+  if (takes_row_ln(a)) return row_ln(*a, s);
   const bool q8 = a->y8 != nullptr;
   if (a->x_dtype == WAM_F32) q8 ? launch_ln<true, true>(a, s) : launch_ln<true, false>(a, s);
   else q8 ? launch_ln<false, true>(a, s) : launch_ln<false, false>(a, s);
