@@ -77,7 +77,7 @@ SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_byte
       if (ks < 1) continue;
       const int64_t rounds = (tiles * ks + cus - 1) / cus, steps = (nk + ks - 1) / ks;
       const int64_t bytes = ks > 1 ? ks * (int64_t)M * seg_n * n_seg * 4 : 0;
-      if (bytes > ws_bytes) continue;
+      if (bytes > ws_bytes || bytes >= INT32_MAX) continue;  // (32-bit offsets in the reduce passes)
       double cost = (double)rounds * (t.round + (double)steps * t.step);
       cost = kLaunch + (cost > hbm ? cost : hbm);
       if (ks > 1) cost += kReduce + kPerMB * 1e-6 * (double)bytes;
@@ -166,11 +166,13 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
   constexpr bool RES = EPI == WAM_EPI_BIAS_GATE_RES || EPI == WAM_EPI_BIAS_RES;
   Raw4 rraw{};
   if constexpr (RES) rraw = ld4_raw(p.res, p.res_f32 != 0, (int64_t)m * p.ldr + n);
-  const f32x4 v = sum_ranges(p.part, p.k_split, (int64_t)p.M * p.part_ld, (int64_t)m * p.part_ld + c);
+  const int off[1] = {(m * p.part_ld + c) * 4};
+  f32x4 v[1];
+  sum_ranges<1>(p, off, v);
   if (bias) widen4_bf16(braw, bv);
   if constexpr (RES) widen4(rraw, p.res_f32 != 0, rv);
   const float no_gate[4] = {0.f, 0.f, 0.f, 0.f};
-  epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v, bv, wsc, no_gate, false, rv);
+  epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v[0], bv, wsc, no_gate, false, rv);
 }
 
 int split_reduce(const LinearParams& p, int wb, hipStream_t s) {

@@ -51,17 +51,20 @@ __global__ __launch_bounds__(kRowThreads) void split_rms_rope_kernel(LinearParam
     const float2 f0 = fp[0], f1 = fp[1];
     fr[c] = make_float4(f0.x, f0.y, f1.x, f1.y);
   }
+  int off[NCH];
+  f32x4 v[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) off[c] = (row * p.part_ld + seg * D + min((tid + kRowThreads * c) * 4, D - 4)) * 4;
+  sum_ranges<NCH>(p, off, v);
   float y[NCH][4], ss = 0.f;
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     const bool in = (tid + kRowThreads * c) * 4 < D;
-    const int n = min((tid + kRowThreads * c) * 4, D - 4);
-    const f32x4 v = sum_ranges(p.part, p.k_split, (int64_t)p.M * p.part_ld, (int64_t)row * p.part_ld + seg * D + n);
     float bv[4];
     widen4(braw[c], false, bv);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      y[c][e] = static_cast<float>(static_cast<bf16>(bias ? v[e] + bv[e] : v[e]));
+      y[c][e] = static_cast<float>(static_cast<bf16>(bias ? v[c][e] + bv[e] : v[c][e]));
       ss += in ? y[c][e] * y[c][e] : 0.f;
     }
   }
@@ -127,6 +130,13 @@ __global__ __launch_bounds__(kRowThreads) void row_ln_kernel(LinearParams p, wam
       gr1[c] = ld4_raw(gm.temb, gf1, g1 + n);
     }
   }
+  f32x4 sums[NCH];
+  if constexpr (SRC != kRowInput) {
+    int off[NCH];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) off[c] = (row * p.part_ld + min((tid + kRowThreads * c) * 4, D - 4)) * 4;
+    sum_ranges<NCH>(p, off, sums);
+  }
   float v[NCH][4], s = 0.f;
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(kRowThreads) void row_ln_kernel(LinearParams p, wam
     const int n = min((tid + kRowThreads * c) * 4, D - 4);
     widen4(xr[c], xf32, v[c]);
     if constexpr (SRC != kRowInput) {
-      const f32x4 y = sum_ranges(p.part, p.k_split, (int64_t)p.M * p.part_ld, (int64_t)row * p.part_ld + n);
+      const f32x4 y = sums[c];
       float bv[4], ga[4], gb[4];
       widen4(br[c], false, bv);
       if constexpr (SRC == kRowGated) {
