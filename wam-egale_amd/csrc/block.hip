@@ -4,7 +4,7 @@
 //   h1  = LN(x) * (1 + scale) + shift                       ln_modulate
 //   qkv = h1 [Wq|Wk|Wv]^T + b                               one GEMM launch
 //   q,k = rope(RMS(q) g_q), rope(RMS(k) g_k)                rms_rope (in place)
-//   [pool bookkeeping]                                       kv_layout
+//   [pool bookkeeping]                                       (a workgroup of the row pass)
 //   a1  = attention(q, [history || k], [history || v])       attention
 //   x1  = x + (a1 Wo^T + bo) * gate                          GEMM + gated residual
 //   [commit new K/V to the pool, update 1/2]                 kv_commit
@@ -25,18 +25,20 @@
 #include <string.h>
 #include <vector>
 #include "gemm_tile.h"
+#include "kv_layout.h"
 
 namespace wam {
 
 int linear(const wam_linear_args*, hipStream_t);
 int mx_dequant_bf16(const void* q, const void* e, void* y, int rows, int cols, hipStream_t s);
 int ln_modulate(const wam_ln_args*, hipStream_t);
-int rms_rope(const wam_rms_rope_args*, hipStream_t);
+int rms_rope(const wam_rms_rope_args*, const wam_kv_layout_args*, hipStream_t);
 int attention(const wam_attention_args*, hipStream_t);
 int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys);
 int64_t linear_workspace_bytes(int M, int seg_n, int n_seg, int K);
 bool linear_norm_in_epilogue(int M, int seg_n, int n_seg, int K, int64_t ws_bytes, bool rope);
 int kv_layout(const wam_kv_layout_args*, hipStream_t);
+int kv_layout_check(const wam_kv_layout_args*);
 int kv_commit(const wam_kv_commit_args*, hipStream_t);
 
 static thread_local char g_error[1024] = "";
@@ -199,7 +201,7 @@ static int context_kv(const wam_block_weights* W, const void* ctx, int rows, voi
   wam_rms_rope_args r{};
   r.x[0] = k; r.y[0] = k; r.gamma[0] = W->w[22]; r.eps[0] = W->eps[6];
   r.ldx = D; r.ldy = D; r.n_tensors = 1; r.rows = rows; r.D = D; r.head_dim = W->head_dim;
-  return rms_rope(&r, s);
+  return rms_rope(&r, nullptr, s);
 }
 
 static int block_forward(const wam_block_args* a, hipStream_t s) {
@@ -349,13 +351,27 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
         wam_rms_rope_args r{};
         r.x[0] = split ? lin : qkv + i * D; r.y[0] = dbg(17 + i); r.gamma[0] = W->w[11 + i]; r.eps[0] = W->eps[3 + i];
         r.ldx = split ? D : 3 * D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
-        WAM_TRY(rms_rope(&r, s));
+        WAM_TRY(rms_rope(&r, nullptr, s));
       }
     }
     return WAM_OK;
   };
   if (!split) WAM_TRY(qk_debug());
   // 3. q/k RMSNorm across heads + RoPE, in place.
+  // 4. Pool bookkeeping: one workgroup's work, independent of the rows, so it
+  //    runs as a workgroup of the same launch (6240 slots: a launch of its own
+  //    took 9.5-11 us, 5 us read only; as a workgroup of the row pass 0.8-1.3
+  //    us of 2 x 16 rows, within the pass from 224 rows on).  Pools whose
+  //    flags do not fit 32 slots per thread of that launch keep their own.
+  wam_kv_layout_args k{};
+  if (cache) {
+    k.mask = a->cache_mask; k.ids = a->cache_id; k.is_pred = a->cache_is_pred; k.pool = a->pool;
+    k.tokens = M; k.update = a->update; k.candidate = candidate ? 1 : 0;
+    k.rows = a->candidate_rows; k.batch = B; k.pool_batch = a->cache_batch;
+    k.hist_slots = slots; k.new_slots = newslots; k.info = info;
+  }
+  const bool kv_rides = cache && a->pool <= kLayoutSlots * 256;
+  if (kv_rides) WAM_TRY(kv_layout_check(&k));
   {
     Scope sc(a->timer, WAM_STAGE_RMS_ROPE, s);
     wam_rms_rope_args r{};
@@ -364,7 +380,8 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     r.ldx = 3 * D; r.ldy = 3 * D; r.n_tensors = 2; r.rows = R; r.D = D;
     r.head_dim = W->head_dim;
     r.freq = a->freq; r.freq_batch = a->freq_batch; r.tokens = M;
-    WAM_TRY(split ? split_rms_rope(sp, r, s) : rms_rope(&r, s));
+    const wam_kv_layout_args* kv = kv_rides ? &k : nullptr;
+    WAM_TRY(split ? split_rms_rope(sp, r, kv, s) : rms_rope(&r, kv, s));
   }
   if (split) WAM_TRY(qk_debug());
   if (a->debug) {
@@ -373,15 +390,9 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
         WAM_HIP(hipMemcpy2DAsync(a->debug[1 + i], D * 2, qkv + i * D, 3 * D * 2, D * 2, R,
                                  hipMemcpyDeviceToDevice, s));
   }
-  // 4. Pool bookkeeping.
   if (cache) {
     Scope sc(a->timer, WAM_STAGE_KV_LAYOUT, s);
-    wam_kv_layout_args k{};
-    k.mask = a->cache_mask; k.ids = a->cache_id; k.is_pred = a->cache_is_pred; k.pool = a->pool;
-    k.tokens = M; k.update = a->update; k.candidate = candidate ? 1 : 0;
-    k.rows = a->candidate_rows; k.batch = B; k.pool_batch = a->cache_batch;
-    k.hist_slots = slots; k.new_slots = newslots; k.info = info;
-    WAM_TRY(kv_layout(&k, s));
+    if (!kv_rides) WAM_TRY(kv_layout(&k, s));
   }
   // 5. Self attention over [history || own].
   {
@@ -459,7 +470,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       wam_rms_rope_args r{};
       r.x[0] = cq; r.y[0] = cq; r.gamma[0] = W->w[21]; r.eps[0] = W->eps[5];
       r.ldx = D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
-      WAM_TRY(split ? split_rms_rope(sp, r, s) : rms_rope(&r, s));
+      WAM_TRY(split ? split_rms_rope(sp, r, nullptr, s) : rms_rope(&r, nullptr, s));
     }
   }
   if (qnorm_fused) {
@@ -472,7 +483,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       wam_rms_rope_args r{};
       r.x[0] = dbg(7); r.y[0] = dbg(7); r.gamma[0] = W->w[21]; r.eps[0] = W->eps[5];
       r.ldx = D; r.ldy = D; r.n_tensors = 1; r.rows = R; r.D = D; r.head_dim = W->head_dim;
-      WAM_TRY(rms_rope(&r, s));
+      WAM_TRY(rms_rope(&r, nullptr, s));
     }
   } else {
     if (split && dbg(20)) WAM_TRY(plain_linear(n2, D, D, 13, -1, dbg(20)));

@@ -53,7 +53,7 @@ int split_reduce(const LinearParams& p, int wb, hipStream_t s);
 // partial sums written, the reduction left to the caller (split_reduce,
 // split_rms_rope or split_ln on *p).  Otherwise nothing is launched.
 int linear_partials(const wam_linear_args* a, hipStream_t s, LinearParams* p, bool* split);
-int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, hipStream_t s);
+int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s);
 int split_ln(const LinearParams& p, const wam_ln_args& l, hipStream_t s);
 // One launch of the four-wave kernel on 224- or 256-row tiles (bf16 or fp8
 // weights); with p.k_split > 1 its partial sums only.

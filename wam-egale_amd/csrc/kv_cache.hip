@@ -21,7 +21,7 @@
 // up to fp32 summation order.  The native reference does the same work in
 // layout_kernel / private_kernel / restore_kernel,
 // 算子研究/wam_ops/baseline/csrc/block.cu:133-227.
-#include "wam_common.h"
+#include "kv_layout.h"
 
 namespace wam {
 
@@ -75,54 +75,23 @@ __device__ inline long long block_reduce_ll(long long v, bool take_max, long lon
   return r;
 }
 
-// Thread t owns the contiguous slots [t * S, t * S + S) (S = ceil(P / 1024)),
-// so every list below is built in ascending slot order by one block scan over
-// per-thread counts.  With MAXS > 0 (S <= MAXS) the thread reads its slots'
-// mask and ids once, all loads issued together, and keeps them in registers
-// through the passes (eviction rounds, next id, history list); read from
-// memory in every pass, each load sat in a branch of its own and cost one
-// round trip.  MAXS == 0 reads memory in every pass (pools beyond 8192
-// slots: 16 slots per thread in registers spilled).
-template <int MAXS>
-__global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout_args a) {
+// Pools beyond 32 slots per thread of the kernel below.  Thread t owns the contiguous slots
+// [t * S, t * S + S) (S = ceil(P / 1024)), so every list below is built in
+// ascending slot order by one block scan over per-thread counts; mask and ids
+// are read from memory in every pass.
+__global__ __launch_bounds__(kLayoutThreads) void kv_layout_large_kernel(wam_kv_layout_args a) {
   __shared__ int sh_i[kLayoutWaves];
   __shared__ long long sh_ll[kLayoutWaves];
   const int tid = threadIdx.x, P = a.pool;
   const int S = (P + kLayoutThreads - 1) / kLayoutThreads;
   const int lo = min(tid * S, P), hi = min(lo + S, P);
-  static_assert(MAXS <= 32, "the valid flags are bits of one word");
-  constexpr int NS = MAXS > 0 ? MAXS : 1;
-  uint32_t mbits = 0;  // bit j: slot lo + j is valid
-  long long idreg[NS];
-  if constexpr (MAXS > 0) {
-    uint8_t mreg[MAXS];
-#pragma unroll
-    for (int j = 0; j < MAXS; ++j) mreg[j] = a.mask[min(lo + j, P - 1)];
-    if (!a.candidate) {
-#pragma unroll
-      for (int j = 0; j < MAXS; ++j) idreg[j] = (long long)a.ids[min(lo + j, P - 1)];
-    }
-#pragma unroll
-    for (int j = 0; j < MAXS; ++j) mbits |= (lo + j < hi && mreg[j] != 0) ? 1u << j : 0u;
-  }
   // slot lo + j of this thread (j < S): valid?  id?
-  auto valid = [&](int j) -> bool {
-    if constexpr (MAXS > 0) return (mbits >> j) & 1u;
-    else return lo + j < hi && a.mask[lo + j] != 0;
-  };
-  auto id_of = [&](int j) -> long long {
-    if constexpr (MAXS > 0) return idreg[j];
-    else return (long long)a.ids[lo + j];
-  };
+  auto valid = [&](int j) -> bool { return lo + j < hi && a.mask[lo + j] != 0; };
+  auto id_of = [&](int j) -> long long { return (long long)a.ids[lo + j]; };
   auto evict = [&](int j) {
-    if constexpr (MAXS > 0) {
-      mbits &= ~(1u << j);
-      idreg[j] = -1;
-    }
     a.mask[lo + j] = 0;
     a.ids[lo + j] = -1;
   };
-  const int NJ = MAXS > 0 ? MAXS : S;  // slots visited per thread (MAXS: unrolled, masked)
   if (a.candidate) {
     // Read only (candidate verification): the history list and its summary
     // in one block pass: per wave a scan of the threads' valid counts and
@@ -135,8 +104,7 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
     for (int b = tid; b < a.batch; b += kLayoutThreads)
       bad |= (a.rows[b] < 0 || a.rows[b] >= a.pool_batch);
     int nv = 0, first = 0x7fffffff, lastv = -1;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < S; ++j)
       if (valid(j)) {
         ++nv;
         first = min(first, lo + j);
@@ -172,8 +140,7 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
       bb |= sh_c[i][3];
     }
     int pv = off + x - nv;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < S; ++j)
       if (valid(j)) a.hist_slots[pv++] = lo + j;
     if (tid == 0) {
       a.info[0] = tv;
@@ -186,22 +153,18 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
   {
     // Eviction of the oldest ids (allocate_slots).
     int nfree = 0;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) nfree += (lo + j < hi && !valid(j)) ? 1 : 0;
+    for (int j = 0; j < S; ++j) nfree += (lo + j < hi && !valid(j)) ? 1 : 0;
     int need = a.tokens - block_sum(nfree, sh_i);
     while (need > 0) {
       long long mn = 0x7fffffffffffffffLL;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < S; ++j)
         if (valid(j) && id_of(j) < mn) mn = id_of(j);
       mn = block_reduce_ll(mn, false, sh_ll);
       int f = 0;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) f += (valid(j) && id_of(j) == mn) ? 1 : 0;
+      for (int j = 0; j < S; ++j) f += (valid(j) && id_of(j) == mn) ? 1 : 0;
       int tot;
       int pos = block_excl_scan(f, sh_i, &tot);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
+      for (int j = 0; j < S; ++j) {
         if (valid(j) && id_of(j) == mn) {
           if (pos < need) evict(j);
           ++pos;
@@ -216,21 +179,16 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
     }
   }
   // Next id over the (post-eviction) valid slots (_next_cache_id).
-  long long next = -1;
-  if (!a.candidate) {
-    long long mx = -1;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      if (valid(j) && id_of(j) > mx) mx = id_of(j);
-    next = block_reduce_ll(mx, true, sh_ll) + 1;
-  }
+  long long mx = -1;
+  for (int j = 0; j < S; ++j)
+    if (valid(j) && id_of(j) > mx) mx = id_of(j);
+  const long long next = block_reduce_ll(mx, true, sh_ll) + 1;
   // History list and new slots, both in ascending slot order.
   int nv = 0, nf = 0;
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
+  for (int j = 0; j < S; ++j) {
     const bool in = lo + j < hi, v = valid(j);
     nv += v ? 1 : 0;
-    nf += (!a.candidate && in && !v) ? 1 : 0;
+    nf += (in && !v) ? 1 : 0;
   }
   int tv, tf;
   int pv = block_excl_scan(nv, sh_i, &tv);
@@ -238,21 +196,19 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
   // Is the history one run of consecutive slots?  (Its first and last valid
   // slots, before this call's new slots are marked.)
   long long first = 0x7fffffffffffffffLL, lastv = -1;
-#pragma unroll
-  for (int j = 0; j < NJ; ++j)
+  for (int j = 0; j < S; ++j)
     if (valid(j)) {
       first = min(first, (long long)(lo + j));
       lastv = max(lastv, (long long)(lo + j));
     }
   first = block_reduce_ll(first, false, sh_ll);
   lastv = block_reduce_ll(lastv, true, sh_ll);
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
+  for (int j = 0; j < S; ++j) {
     const int i = lo + j;
     if (i >= hi) continue;
     const bool v = valid(j);
     if (v) a.hist_slots[pv++] = i;
-    if (!a.candidate && !v) {
+    if (!v) {
       if (pf < a.tokens) {
         a.new_slots[pf] = i;
         a.mask[i] = a.update != 0 ? 1 : 0;
@@ -269,7 +225,11 @@ __global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout
   }
 }
 
-int kv_layout(const wam_kv_layout_args* a, hipStream_t s) {
+__global__ __launch_bounds__(kLayoutThreads) void kv_layout_kernel(wam_kv_layout_args a) {
+  kv_layout_pool<kLayoutThreads>(a);
+}
+
+int kv_layout_check(const wam_kv_layout_args* a) {
   WAM_REQUIRE(a != nullptr, "wam_kv_layout: null args");
   WAM_REQUIRE(a->mask && a->ids && a->is_pred && a->hist_slots && a->info,
               "wam_kv_layout: null pool state");
@@ -284,9 +244,13 @@ int kv_layout(const wam_kv_layout_args* a, hipStream_t s) {
     WAM_REQUIRE(a->tokens >= 1 && a->tokens <= a->pool,
                 "wam_kv_layout: %d new tokens do not fit a pool of %d slots", a->tokens, a->pool);
   }
-  const int S = (a->pool + kLayoutThreads - 1) / kLayoutThreads;
-  if (S <= 8) hipLaunchKernelGGL(kv_layout_kernel<8>, dim3(1), dim3(kLayoutThreads), 0, s, *a);
-  else hipLaunchKernelGGL(kv_layout_kernel<0>, dim3(1), dim3(kLayoutThreads), 0, s, *a);
+  return WAM_OK;
+}
+
+int kv_layout(const wam_kv_layout_args* a, hipStream_t s) {
+  WAM_TRY(kv_layout_check(a));
+  if (a->pool <= kLayoutSlots * kLayoutThreads) hipLaunchKernelGGL(kv_layout_kernel, dim3(1), dim3(kLayoutThreads), 0, s, *a);
+  else hipLaunchKernelGGL(kv_layout_large_kernel, dim3(1), dim3(kLayoutThreads), 0, s, *a);
   WAM_LAUNCHED("kv_layout_kernel");
   return WAM_OK;
 }

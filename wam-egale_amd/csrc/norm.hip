@@ -12,7 +12,7 @@
 // RMSNorm+RoPE follows model.py:609-623: RMSNorm over the full D-wide row
 // (all heads), times the affine weight, then the complex rotation of pair
 // (2j, 2j+1) of every head by freq[t, j]; baseline/csrc/block.cu:103-118.
-#include "wam_common.h"
+#include "kv_layout.h"
 
 namespace wam {
 
@@ -293,10 +293,13 @@ int ln_modulate(const wam_ln_args* a, hipStream_t s) {
 }
 
 // ------------------------------------------------------- RMSNorm + RoPE
-template <int CH>
-__global__ __launch_bounds__(256) void rms_rope_kernel(wam_rms_rope_args a) {
+// KV: the first workgroup does the KV pool's bookkeeping instead.
+template <int CH, bool KV>
+__global__ __launch_bounds__(256) void rms_rope_kernel(wam_rms_rope_args a, wam_kv_layout_args kv) {
+  if constexpr (KV)
+    if (blockIdx.x == 0) return kv_layout_pool<256>(kv);
   const int lane = threadIdx.x & 63;
-  const int64_t job = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t job = (int64_t)(blockIdx.x - (KV ? 1 : 0)) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (job >= (int64_t)a.rows * a.n_tensors) return;
   const int tsel = (int)(job % a.n_tensors);
   const int64_t row = job / a.n_tensors;
@@ -378,7 +381,17 @@ __global__ __launch_bounds__(256) void rms_rope_kernel(wam_rms_rope_args a) {
   }
 }
 
-int rms_rope(const wam_rms_rope_args* a, hipStream_t s) {
+template <int CH>
+static void launch_rms_rope(const wam_rms_rope_args& a, const wam_kv_layout_args* kv, hipStream_t s) {
+  const int64_t jobs = (int64_t)a.rows * a.n_tensors;
+  const dim3 grid((unsigned)((jobs + 3) / 4 + (kv ? 1 : 0))), block(256);
+  if (kv) hipLaunchKernelGGL((rms_rope_kernel<CH, true>), grid, block, 0, s, a, *kv);
+  else hipLaunchKernelGGL((rms_rope_kernel<CH, false>), grid, block, 0, s, a, wam_kv_layout_args{});
+}
+
+// kv (may be null): the KV pool's bookkeeping, done by one workgroup of the
+// launch (pools of up to kLayoutSlots * 256 slots).
+int rms_rope(const wam_rms_rope_args* a, const wam_kv_layout_args* kv, hipStream_t s) {
   WAM_REQUIRE(a != nullptr, "wam_rms_rope: null args");
   WAM_REQUIRE(a->n_tensors == 1 || a->n_tensors == 2, "wam_rms_rope: n_tensors must be 1 or 2");
   WAM_REQUIRE(a->D > 0 && a->D % 8 == 0 && a->D <= 4096, "wam_rms_rope: D=%d unsupported", a->D);
@@ -394,14 +407,12 @@ int rms_rope(const wam_rms_rope_args* a, hipStream_t s) {
                 "wam_rms_rope: freq batch %d / tokens %d contract", a->freq_batch, a->tokens);
   }
   if (a->rows == 0) return WAM_OK;
-  const int64_t jobs = (int64_t)a->rows * a->n_tensors;
-  const dim3 grid((unsigned)((jobs + 3) / 4)), block(256);
   const int ch = (a->D / 8 + 63) / 64;
-  if (ch <= 1) hipLaunchKernelGGL(rms_rope_kernel<1>, grid, block, 0, s, *a);
-  else if (ch <= 2) hipLaunchKernelGGL(rms_rope_kernel<2>, grid, block, 0, s, *a);
-  else if (ch <= 3) hipLaunchKernelGGL(rms_rope_kernel<3>, grid, block, 0, s, *a);
-  else if (ch <= 6) hipLaunchKernelGGL(rms_rope_kernel<6>, grid, block, 0, s, *a);
-  else hipLaunchKernelGGL(rms_rope_kernel<8>, grid, block, 0, s, *a);
+  if (ch <= 1) launch_rms_rope<1>(*a, kv, s);
+  else if (ch <= 2) launch_rms_rope<2>(*a, kv, s);
+  else if (ch <= 3) launch_rms_rope<3>(*a, kv, s);
+  else if (ch <= 6) launch_rms_rope<6>(*a, kv, s);
+  else launch_rms_rope<8>(*a, kv, s);
   WAM_LAUNCHED("rms_rope_kernel");
   return WAM_OK;
 }
@@ -412,5 +423,5 @@ extern "C" int wam_ln_modulate(const wam_ln_args* args, void* stream) {
   return wam::ln_modulate(args, static_cast<hipStream_t>(stream));
 }
 extern "C" int wam_rms_rope(const wam_rms_rope_args* args, void* stream) {
-  return wam::rms_rope(args, static_cast<hipStream_t>(stream));
+  return wam::rms_rope(args, nullptr, static_cast<hipStream_t>(stream));
 }

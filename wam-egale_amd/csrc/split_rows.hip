@@ -6,6 +6,7 @@
 // the reduce and the LayerNorm, 5.5 us together).  The same kernel without
 // partial sums is the LayerNorm of few rows.
 #include "gemm_tile.h"
+#include "kv_layout.h"
 
 namespace wam {
 
@@ -24,12 +25,16 @@ __device__ inline float block_sum(float v, float (*sh)[4], int slot) {
 // q/k/v: y = bf16(sum + bias) as the projection rounds it; segments with a
 // gamma (s < r.n_tensors) are then normalised over the row and rotated, as
 // rms_rope_kernel does.  NCH chunks of 4 columns per thread, 1024 apart.
-template <int NCH>
-__global__ __launch_bounds__(kRowThreads) void split_rms_rope_kernel(LinearParams p, wam_rms_rope_args r) {
+// KV: the first workgroup does the KV pool's bookkeeping instead.
+template <int NCH, bool KV>
+__global__ __launch_bounds__(kRowThreads) void split_rms_rope_kernel(LinearParams p, wam_rms_rope_args r,
+                                                                     wam_kv_layout_args kv) {
   __shared__ float sh[1][4];
-  const int tid = threadIdx.x, D = p.seg_n;
-  const int row = __builtin_amdgcn_readfirstlane(blockIdx.x / p.n_seg_count);
-  const int seg = __builtin_amdgcn_readfirstlane(blockIdx.x - row * p.n_seg_count);
+  if constexpr (KV)
+    if (blockIdx.x == 0) return kv_layout_pool<kRowThreads>(kv);
+  const int tid = threadIdx.x, D = p.seg_n, job = blockIdx.x - (KV ? 1 : 0);
+  const int row = __builtin_amdgcn_readfirstlane(job / p.n_seg_count);
+  const int seg = __builtin_amdgcn_readfirstlane(job - row * p.n_seg_count);
   const bf16* bias = seg == 0 ? p.bias[0] : (seg == 1 ? p.bias[1] : p.bias[2]);
   bf16* out = static_cast<bf16*>(seg == 0 ? p.out[0] : (seg == 1 ? p.out[1] : p.out[2])) + (int64_t)row * p.ldo;
   const bool norm = seg < r.n_tensors;
@@ -210,13 +215,19 @@ __global__ __launch_bounds__(kRowThreads) void row_ln_kernel(LinearParams p, wam
   }
 }
 
-int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, hipStream_t s) {
-  const dim3 grid((unsigned)(p.M * p.n_seg_count)), block(kRowThreads);
+template <int NCH>
+static void launch_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s) {
+  const dim3 grid((unsigned)(p.M * p.n_seg_count + (kv ? 1 : 0))), block(kRowThreads);
+  if (kv) hipLaunchKernelGGL((split_rms_rope_kernel<NCH, true>), grid, block, 0, s, p, r, *kv);
+  else hipLaunchKernelGGL((split_rms_rope_kernel<NCH, false>), grid, block, 0, s, p, r, wam_kv_layout_args{});
+}
+
+int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s) {
   switch ((p.seg_n + 1023) / 1024) {
-    case 1: hipLaunchKernelGGL(split_rms_rope_kernel<1>, grid, block, 0, s, p, r); break;
-    case 2: hipLaunchKernelGGL(split_rms_rope_kernel<2>, grid, block, 0, s, p, r); break;
-    case 3: hipLaunchKernelGGL(split_rms_rope_kernel<3>, grid, block, 0, s, p, r); break;
-    default: hipLaunchKernelGGL(split_rms_rope_kernel<4>, grid, block, 0, s, p, r); break;
+    case 1: launch_rms_rope<1>(p, r, kv, s); break;
+    case 2: launch_rms_rope<2>(p, r, kv, s); break;
+    case 3: launch_rms_rope<3>(p, r, kv, s); break;
+    default: launch_rms_rope<4>(p, r, kv, s); break;
   }
   WAM_LAUNCHED("split_rms_rope_kernel");
   return WAM_OK;
