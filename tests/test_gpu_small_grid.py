@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from oracle.fp8 import dequantize_rows
+from oracle.fp8 import dequantize_mx32, dequantize_rows, quantize_mx32
 from oracle.metrics import assert_close
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +94,53 @@ def test_without_and_with_a_small_workspace(dev):
         _lib.check(h.wam_linear(ctypes.byref(a), None), "wam_linear")
         torch.cuda.synchronize()
         assert_close(out, ref, _ulp(ref), 0.99999, f"workspace of {nbytes} bytes")
+
+
+# fp8 activations: 128-row tiles (up to 128 rows in one, 129 in two), 224-row
+# ones (780 x 3072 x 14336), one k-tile, nine over the ranges, and whole k with
+# 128-row tiles (2325); without a workspace one range, with one the plan's.
+@pytest.mark.parametrize("M,K,N", [(1, 128, 256), (32, 3072, 14336), (128, 14336, 3072), (129, 14336, 3072),
+                                   (225, 1152, 512), (780, 3072, 14336), (780, 14336, 3072), (2325, 14336, 3072)])
+@pytest.mark.parametrize("room", [False, True])
+def test_fp8_activations(dev, M, K, N, room):
+    from wam_ops import _lib, ops
+    x, w, b = _randn((M, K), dev, 1), _randn((N, K), dev, 2, 0.02), _randn((N,), dev, 3)
+    qw, sw = ops.quantize_fp8_rows(w)
+    wd = dequantize_rows(qw.cpu(), sw.cpu()).to(dev).t()
+    ws = torch.empty(32 * M * N * 4 if room else 1, dtype=torch.uint8, device=dev)
+
+    def run(q, out, epi, **kw):
+        a = _lib.LinearArgs()
+        a.a, a.lda, a.M, a.K, a.n_seg, a.seg_n, a.ldw, a.ldo = q.data_ptr(), K, M, K, 1, N, K, N
+        a.w[0], a.out[0], a.bias[0], a.w_dtype, a.w_scale[0] = qw.data_ptr(), out.data_ptr(), b.data_ptr(), _lib.WAM_FP8, sw.data_ptr()
+        a.epilogue, a.a_dtype = epi, _lib.WAM_FP8
+        for k, v in kw.items():
+            setattr(a, k, v)
+        if room:
+            a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        _lib.check(_lib.lib().wam_linear(ctypes.byref(a), None), "wam_linear")
+        torch.cuda.synchronize()
+        return out
+
+    q, sx = ops.quantize_fp8_rows(x)
+    ref = dequantize_rows(q.cpu(), sx.cpu()).to(dev) @ wd + b.float()
+    y = run(q, torch.zeros(M, N, dtype=torch.bfloat16, device=dev), ops.EPI_BIAS, a_scale=sx.data_ptr())
+    assert_close(y, ref, _ulp(ref), 0.99999, f"fp8 rows, bias {M}x{K}x{N}")
+    gelu = torch.nn.functional.gelu(ref, approximate="tanh")
+    e = torch.zeros(M, N // 32, dtype=torch.uint8, device=dev)
+    y = run(q, torch.zeros(M, N, dtype=torch.float8_e4m3fn, device=dev), ops.EPI_BIAS_GELU, a_scale=sx.data_ptr(),
+            out_dtype=_lib.WAM_FP8_MX, out_block_scale=e.data_ptr())
+    d = dequantize_mx32(y.cpu(), e.cpu()).to(dev)
+    # half an e4m3 step (2^-4 of the value, 2^-10 of a subnormal's block scale) and fp32 summation order
+    step = torch.maximum(gelu.abs() * 2.0 ** -4, torch.exp2(e.float() - 137).repeat_interleave(32, 1))
+    assert ((d - gelu).abs() <= step + 2e-3).all()
+    q, ex = quantize_mx32(x.float().cpu())
+    ref = dequantize_mx32(q, ex).to(dev) @ wd + b.float()
+    q, ex = q.to(dev), ex.to(dev)
+    res = _randn((M, N), dev, 4, 1.0, torch.float32)
+    table, temb = _randn((1, 6, N), dev, 5, 0.3, torch.float32), _randn((1, M, 6, N), dev, 6, 0.3)
+    ref = res + ref * (table[:, 5] + temb[0, :, 5].float())
+    y = run(q, torch.zeros(M, N, device=dev), ops.EPI_BIAS_GATE_RES, a_dtype=_lib.WAM_FP8_MX, a_block_scale=ex.data_ptr(),
+            res=res.data_ptr(), ldr=N, res_dtype=_lib.WAM_F32, out_dtype=_lib.WAM_F32,
+            gate=ops.modulation(table, temb, M), gate_index=5)
+    assert_close(y, ref, 2e-3, 0.99999, f"MX gated residual {M}x{K}x{N}")

@@ -93,18 +93,18 @@ __device__ __forceinline__ void w4_sched() {
 // 32 k instead of a row scale, applied as the MFMA's block scales.
 template <int EPI, int RF32, int OF32, int TM, int WB = 2, bool F8MM = false, bool AMX = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
-  static_assert(TM == 256 || TM == 224, "tile rows");
+  static_assert(TM == 256 || TM == 224 || (TM == 128 && F8MM), "tile rows");
   static_assert(WB == 2 || WB == 1, "weight bytes");
   constexpr bool MXO = OF32 == 2;  // e4m3 output with e8m0 exponents per 32 columns
-  static_assert(!F8MM || (WB == 2 && TM == 224), "fp8 MFMA: 224-row tiles");
-  static_assert(!F8MM || AMX || EPI == WAM_EPI_BIAS || EPI == WAM_EPI_BIAS_GELU,
+  static_assert(!F8MM || (WB == 2 && TM != 256), "fp8 MFMA: 224- or 128-row tiles");
+  static_assert(!F8MM || AMX || EPI == WAM_EPI_BIAS || EPI == WAM_EPI_BIAS_GELU || EPI == kEpiPartial,
                 "fp8 MFMA with per-row activation scales: bias or GELU epilogue");
   static_assert(!AMX || (F8MM && !MXO && EPI != WAM_EPI_BIAS_GELU), "MX activations: fp8 MFMA, bf16 output");
   static_assert(!MXO || (F8MM && !AMX && (EPI == WAM_EPI_BIAS || EPI == WAM_EPI_BIAS_GELU)),
                 "MX output: fp8 MFMA with per-row activation scales, bias or GELU");
   constexpr int AE = F8MM ? 1 : 2;        // bytes per A element
   constexpr int WE = F8MM ? 1 : WB;       // bytes per W element
-  constexpr int MB = TM == 256 ? 4 : 7;   // 32-row m-blocks per wave
+  constexpr int MB = TM == 256 ? 4 : TM / 32;  // 32-row m-blocks per wave
   constexpr int NB = TM == 256 ? 4 : 2;   // 32-column n-blocks per wave
   constexpr int WGN = TM == 256 ? 2 : 4;  // waves along n
   constexpr int LA = TM / 32;             // A staging loads per thread and k-step
@@ -227,15 +227,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
   };
   // AMX: the e8m0 exponents of the A tile's rows for a k-step (4 bytes =
   // 4 blocks of 32 per row) ride with the stage, thread t loading row t
-  // into bytes 28672 + 4 t (free: the A rows end at 28672, W starts at
-  // 32768).  Lane half h supplies the scale of MFMA block h, i.e. of the
+  // into bytes 128 TM + 4 t (free: the A rows end there, W starts at 32768).  Lane half h supplies the scale of MFMA block h, i.e. of the
   // k-step's block 2 s + h: its rows' words shifted right by 8 h hold that
   // of sub-step 0 in byte 0 and that of sub-step 1 in byte 2, which the
   // MFMA's operand select picks.
-  constexpr int kScl = 28672;
+  constexpr int kScl = TM * 128;
   const uint32_t ldsc = (uint32_t)p.K / 32u;  // exponent bytes per A row
   const __amdgpu_buffer_rsrc_t rsc =
-      AMX ? make_rsrc(p.abscale + (int64_t)m0 * ldsc, (uint32_t)(p.M - m0) * ldsc) : make_rsrc(p.a, 0u);
+      AMX ? make_rsrc(p.abscale + (int64_t)m0 * ldsc + kb * 4, (uint32_t)(p.M - m0) * ldsc - (uint32_t)kb * 4u)
+          : make_rsrc(p.a, 0u);
   uint32_t ssc = 0;
   uint32_t scw[2][MB];
   auto rd8 = [&](const char* buf, int s, int f, int par) {
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
   // segment's tiles all take one), so no per-row branch remains.
   auto rounds = [&](auto nrm_c, auto rope_c) {
     round(std::integral_constant<int, 0>{}, nrm_c, rope_c);
-    round(std::integral_constant<int, 1>{}, nrm_c, rope_c);
+    if constexpr (TM > 128) round(std::integral_constant<int, 1>{}, nrm_c, rope_c);
   };
   using F = std::false_type;
   using T = std::true_type;
@@ -970,13 +970,51 @@ static bool uses_big_tiles(int M, int seg_n, int n_seg) {
   return seg_n % 256 == 0 && big_tiles >= 200;
 }
 
+// Tile rows (128 or 224) and k ranges of an fp8-activation launch, by the
+// small-grid plan's cost model: rounds of round + steps * step us, steps being
+// 128-deep and a step's time rising with the share of the chip at work (it
+// loads 48 or 60 KB), and the reduce pass.  Measured, weights cold, against
+// 224-row tiles over the whole k (us; F1 is K 3072 to N 14336 with GELU and
+// an MX output, F2 back with a residual; the model is within 15% of these):
+//   32 rows   F1 32 -> 17, F2 98 -> 18      780 rows  F1 50 (224), F2 123 -> 51
+//   224 rows  F1 47 -> 29, F2 156 -> 28     1560 rows F1 97 (224), F2 136 -> 79
+//   400 rows  F1 47 -> 35, F2 142 -> 36     2325 rows F1 141 (224), F2 123 -> 116
+// Ranges are as many as the workspace holds, at most.
+static SplitPlan f8mm_plan(int M, int N, int K, int64_t ws_bytes) {
+  struct { int tm; double round, step, share; } const tiles[2] = {{128, 6.0, 0.78, 0.20}, {224, 11.0, 0.70, 0.65}};
+  const int cus = device_cu_count(), nk = K / 128;
+  const int64_t plane = (int64_t)M * N * 4;
+  SplitPlan best{224, 1};
+  double best_cost = 1e30;
+  for (const auto& t : tiles) {
+    const int64_t n = (int64_t)((M + t.tm - 1) / t.tm) * (N / 256);
+    const int64_t cand[3] = {1, cus / n, 2 * cus / n};
+    for (int64_t ks : cand) {
+      const int64_t most[3] = {32, nk, (ws_bytes < INT32_MAX ? ws_bytes : INT32_MAX - 1) / plane};
+      for (int64_t m : most) ks = ks < m ? ks : m;
+      if (ks < 1) ks = 1;
+      const int64_t rounds = (n * ks + cus - 1) / cus, steps = (nk + ks - 1) / ks;
+      const double used = n * ks < cus ? (double)(n * ks) / cus : 1.0;
+      double cost = kSmallLaunch + (double)rounds * (t.round + (double)steps * (t.step + t.share * used));
+      if (ks > 1) cost += split_reduce_us(ks * plane);
+      if (cost < best_cost - 1e-9) best_cost = cost, best = SplitPlan{t.tm, (int)ks};
+    }
+  }
+  return best;
+}
+
 int64_t linear_workspace_bytes(int M, int seg_n, int n_seg, int K) {
   if (M < 1 || seg_n < 1 || K < 1) return 0;
   if (!uses_big_tiles(M, seg_n, n_seg)) {
-    // bf16 weights (fp8 ones plan their own ranges within it)
+    // bf16 weights (fp8 operands plan their own ranges within it)
     return K % 64 == 0 ? split_plan_bytes(split_plan(M, seg_n, n_seg, K, 2, INT64_MAX), M, seg_n, n_seg) : 0;
   }
   return plan_workspace(gemm_plan(M, seg_n, n_seg, K, device_cu_count(), INT64_MAX), M, seg_n);
+}
+
+// What a launch with fp8 activations can use.
+int64_t linear_f8mm_bytes(int M, int N, int K) {
+  return N % 256 == 0 && K % 128 == 0 ? split_plan_bytes(f8mm_plan(M, N, K, INT64_MAX), M, N, 1) : 0;
 }
 
 // Whether linear() applies the q/k-norm epilogue inside its one launch for
@@ -989,6 +1027,32 @@ bool linear_norm_in_epilogue(int M, int seg_n, int n_seg, int K, int64_t ws_byte
   if (w4_t224_wins(M, seg_n, n_seg, K, cus, ws_bytes)) return true;
   if (t320_one_round(M, seg_n, n_seg, K, cus, ws_bytes)) return !rope;
   return gemm_plan(M, seg_n, n_seg, K, cus, ws_bytes).kind == 0;
+}
+
+// fp8 activations: TM-row tiles, or the partial sums of their k ranges.
+template <int TM>
+static void launch_f8mm(LinearParams& p, bool amx, bool mxo, hipStream_t s) {
+  p.m_tiles = (p.M + TM - 1) / TM;
+  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles * p.k_split)), block(256);
+#define WAM_F8MM(E, RF, OF, MX) hipLaunchKernelGGL((gemm_w4_kernel<E, RF, OF, TM, 2, true, MX>), grid, block, 0, s, p)
+  if (p.k_split > 1) {
+    if (amx) WAM_F8MM(kEpiPartial, 0, 0, true);
+    else WAM_F8MM(kEpiPartial, 0, 0, false);
+  } else if (amx) {
+    if (p.epi == WAM_EPI_BIAS) WAM_F8MM(WAM_EPI_BIAS, 0, 0, true);
+    else if (p.epi == WAM_EPI_BIAS_GATE_RES && p.res_f32 && p.out_f32) WAM_F8MM(WAM_EPI_BIAS_GATE_RES, 1, 1, true);
+    else if (p.epi == WAM_EPI_BIAS_GATE_RES && p.res_f32) WAM_F8MM(WAM_EPI_BIAS_GATE_RES, 1, 0, true);
+    else if (p.epi == WAM_EPI_BIAS_GATE_RES) WAM_F8MM(WAM_EPI_BIAS_GATE_RES, 0, 0, true);
+    else if (p.res_f32) WAM_F8MM(WAM_EPI_BIAS_RES, 1, 0, true);
+    else WAM_F8MM(WAM_EPI_BIAS_RES, 0, 0, true);
+  } else if (p.epi == WAM_EPI_BIAS) {
+    if (mxo) WAM_F8MM(WAM_EPI_BIAS, 0, 2, false);
+    else WAM_F8MM(WAM_EPI_BIAS, 0, 0, false);
+  } else {
+    if (mxo) WAM_F8MM(WAM_EPI_BIAS_GELU, 0, 2, false);
+    else WAM_F8MM(WAM_EPI_BIAS_GELU, 0, 0, false);
+  }
+#undef WAM_F8MM
 }
 
 // The contract of a call, and its launch parameters.
@@ -1118,35 +1182,18 @@ int linear(const wam_linear_args* a, hipStream_t s) {
     WAM_REQUIRE(a->n_seg == 1 && a->seg_n % 256 == 0 && a->K % 128 == 0,
                 "wam_linear: fp8 activations need one segment, N a multiple of 256 and K of 128 (N=%d K=%d)",
                 a->seg_n, a->K);
-    p.ascale = a->a_scale;
-    p.abscale = static_cast<const uint8_t*>(a->a_block_scale);
-    p.oscale = static_cast<uint8_t*>(a->out_block_scale);
+    p.ascale = a8 ? a->a_scale : nullptr;
+    p.abscale = amx ? static_cast<const uint8_t*>(a->a_block_scale) : nullptr;
+    p.oscale = mxo ? static_cast<uint8_t*>(a->out_block_scale) : nullptr;
     p.n_tiles_per_seg = a->seg_n / 256;
-    p.m_tiles = (a->M + 223) / 224;
     p.n_tiles = p.n_tiles_per_seg;
-    const dim3 grid((unsigned)(p.m_tiles * p.n_tiles));
-    if (amx) {
-      if (a->epilogue == WAM_EPI_BIAS)
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS, 0, 0, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-      else if (a->epilogue == WAM_EPI_BIAS_GATE_RES && p.res_f32 && p.out_f32)
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_GATE_RES, 1, 1, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-      else if (a->epilogue == WAM_EPI_BIAS_GATE_RES && p.res_f32)
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_GATE_RES, 1, 0, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-      else if (a->epilogue == WAM_EPI_BIAS_GATE_RES)
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_GATE_RES, 0, 0, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-      else if (p.res_f32)
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_RES, 1, 0, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-      else
-        hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_RES, 0, 0, 224, 2, true, true>), grid, dim3(256), 0, s, p);
-    } else if (a->epilogue == WAM_EPI_BIAS) {
-      if (mxo) hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS, 0, 2, 224, 2, true>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS, 0, 0, 224, 2, true>), grid, dim3(256), 0, s, p);
-    } else {
-      if (mxo) hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_GELU, 0, 2, 224, 2, true>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((gemm_w4_kernel<WAM_EPI_BIAS_GELU, 0, 0, 224, 2, true>), grid, dim3(256), 0, s, p);
-    }
+    p.part_ld = a->seg_n;
+    const SplitPlan g = f8mm_plan(a->M, a->seg_n, a->K, ws_bytes);
+    p.k_split = g.ks;
+    if (g.tile == 128) launch_f8mm<128>(p, amx, mxo, s);
+    else launch_f8mm<224>(p, amx, mxo, s);
     WAM_LAUNCHED("gemm_w4_kernel (fp8 MFMA)");
-    return WAM_OK;
+    return g.ks > 1 ? split_reduce(p, 1, s) : WAM_OK;
   }
   WAM_REQUIRE(!mxo, "wam_linear: an MX output needs fp8 activations with row scales");
   if (f8) {

@@ -28,10 +28,10 @@ using Small64f8 = GemmCfg<64, 128, 64, 1, 4, 5, 1, 0, 1>;
 using Small128f8 = GemmCfg<128, 128, 64, 2, 4, 5, 1, 0, 1>;
 using Small256f8 = GemmCfg<256, 128, 64, 4, 2, 3, 1, 0, 1>;
 
-// Cost model, in us: kLaunch + rounds * (round + steps * step), rounds being
+// Cost model, in us: kSmallLaunch + rounds * (round + steps * step), rounds being
 // dispatch rounds of one workgroup per CU and steps the 64-deep k-steps of
 // one range; at least the weights' time from HBM; and for several ranges the
-// reduce pass, kReduce + kPerMB per MB of partial sums (written and read).
+// reduce pass (split_reduce_us of the partial sums' bytes, written and read).
 // Fitted to 34 shapes (96 to 2325 rows, K 1536 to 14336, N 1536 to 14336, 1
 // to 32 ranges, weights cold): 6% rms, and the plan it picks is within 3% of
 // the fastest measured one but for 400 x 3072 x 14336 (8%) and 224 x 9216 x
@@ -49,7 +49,7 @@ constexpr TileCost kTiles[] = {
     {256, 128, 2.7, 0.81}, {128, 256, 3.1, 0.82}, {224, 256, 4.7, 1.05},  {256, 256, 4.4, 1.21},
 };
 constexpr int kTile32 = 0, kTile192 = 3, kTileN256 = 5, kTileW224 = 6, kTileCount = 8;
-constexpr double kLaunch = 2.6, kReduce = 4.1, kPerMB = 0.28, kHbmBytesPerUs = 6.6e6;
+constexpr double kHbmBytesPerUs = 6.6e6;
 constexpr int kMaxRanges = 32;
 
 SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_bytes) {
@@ -79,8 +79,8 @@ SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_byte
       const int64_t bytes = ks > 1 ? ks * (int64_t)M * seg_n * n_seg * 4 : 0;
       if (bytes > ws_bytes || bytes >= INT32_MAX) continue;  // (32-bit offsets in the reduce passes)
       double cost = (double)rounds * (t.round + (double)steps * t.step);
-      cost = kLaunch + (cost > hbm ? cost : hbm);
-      if (ks > 1) cost += kReduce + kPerMB * 1e-6 * (double)bytes;
+      cost = kSmallLaunch + (cost > hbm ? cost : hbm);
+      if (ks > 1) cost += split_reduce_us(bytes);
       if (cost < best_cost - 1e-9) best_cost = cost, best = SplitPlan{c, (int)ks};
     }
   }
@@ -146,8 +146,10 @@ int split_tiles(LinearParams& p, const SplitPlan& g, int wb, hipStream_t s) {
 
 // ------------------------------------------------------------------ reduce
 // The launch's epilogue over the partial sums, one thread per 4 consecutive
-// outputs of one segment.  W1: fp8 weights (per-column scales).
-template <int EPI, bool W1>
+// outputs of one segment.  W1: fp8 weights (per-column scales).  A8: fp8
+// activations with row scales; MXO: e4m3 output with an exponent per 32
+// columns (8 lanes), as the four-wave kernel writes it.
+template <int EPI, bool W1, bool A8 = false, bool MXO = false>
 __global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
   const int q4 = p.part_ld / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -171,6 +173,27 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
   sum_ranges<1>(p, off, v);
   if (bias) widen4_bf16(braw, bv);
   if constexpr (RES) widen4(rraw, p.res_f32 != 0, rv);
+  if constexpr (A8) {
+    const float sr = p.ascale[m];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wsc[e] = sr * wsc[e];
+  }
+  if constexpr (MXO) {
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = v[0][e] * wsc[e] + bv[e];
+      if constexpr (EPI == WAM_EPI_BIAS_GELU) y[e] = gelu_tanh(y[e]);
+    }
+    const int X = mx_exponent(max8_lanes(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])))));
+    const float inv = __uint_as_float((uint32_t)(127 - X) << 23);
+    int pk = 0;
+    pk = __builtin_amdgcn_cvt_pk_fp8_f32(y[0] * inv, y[1] * inv, pk, false);
+    pk = __builtin_amdgcn_cvt_pk_fp8_f32(y[2] * inv, y[3] * inv, pk, true);
+    *reinterpret_cast<int*>(static_cast<uint8_t*>(out) + (int64_t)m * p.ldo + n) = pk;
+    if ((threadIdx.x & 7) == 0) p.oscale[(int64_t)m * (p.seg_n / 32) + n / 32] = (uint8_t)(X + 127);
+    return;
+  }
   const float no_gate[4] = {0.f, 0.f, 0.f, 0.f};
   epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v[0], bv, wsc, no_gate, false, rv);
 }
@@ -181,6 +204,16 @@ int split_reduce(const LinearParams& p, int wb, hipStream_t s) {
 #define WAM_REDUCE(E)                                                                             \
   if (w1) hipLaunchKernelGGL((split_reduce_kernel<E, true>), grid, block, 0, s, p);               \
   else hipLaunchKernelGGL((split_reduce_kernel<E, false>), grid, block, 0, s, p)
+  if (p.ascale) {  // bias or GELU, whole 256-column tiles
+    const bool gelu = p.epi == WAM_EPI_BIAS_GELU, mxo = p.oscale != nullptr;
+    auto kernel = gelu ? (mxo ? split_reduce_kernel<WAM_EPI_BIAS_GELU, true, true, true>
+                              : split_reduce_kernel<WAM_EPI_BIAS_GELU, true, true, false>)
+                       : (mxo ? split_reduce_kernel<WAM_EPI_BIAS, true, true, true>
+                              : split_reduce_kernel<WAM_EPI_BIAS, true, true, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, p);
+    WAM_LAUNCHED("split_reduce_kernel");
+    return WAM_OK;
+  }
   switch (p.epi) {
     case WAM_EPI_BIAS: WAM_REDUCE(WAM_EPI_BIAS); break;
     case WAM_EPI_BIAS_GELU: WAM_REDUCE(WAM_EPI_BIAS_GELU); break;

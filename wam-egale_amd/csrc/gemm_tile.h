@@ -41,6 +41,9 @@ struct LinearParams {
   uint8_t* oscale;
 };
 
+// Cost of a launch and of the reduce pass over `bytes` of partial sums, us.
+constexpr double kSmallLaunch = 2.6;
+inline double split_reduce_us(int64_t bytes) { return 4.1 + 0.28e-6 * (double)bytes; }
 // Tile (an index into the small-grid plan's table) and k ranges of a launch.
 struct SplitPlan {
   int tile, ks;
