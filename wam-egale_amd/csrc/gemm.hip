@@ -415,6 +415,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
   // most two consecutive modulation rows (samples or latent frames): gate
   // before tile row gate_split, gate2 from there on; otherwise per row.
   float gate[4] = {0.f, 0.f, 0.f, 0.f}, gate2[4] = {0.f, 0.f, 0.f, 0.f};
+  Raw4 gtab{};
   bool gate_held = false;
   int gate_split = 0;
   if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
@@ -424,6 +425,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
     gate_split = (int)(temb_first_row(p.gate, tr1) - m0);
     ld_mod4(p.gate, p.mod_d, m0, p.gate_index, n + p.n_off, gate);
     ld_mod4(p.gate, p.mod_d, m_last, p.gate_index, n + p.n_off, gate2);
+    gtab = ld4_raw(p.gate.table, p.gate.table_dtype == WAM_F32, (int64_t)p.gate_index * p.mod_d + n + p.n_off);
   }
   constexpr bool RES = EPI == WAM_EPI_BIAS_GATE_RES || EPI == WAM_EPI_BIAS_RES;
   constexpr bool PART = EPI == kEpiPartial;
@@ -578,10 +580,21 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
         const int lrw = rr & 63;
         vv[k8] = *reinterpret_cast<const f32x4*>(buf + lrw * 1024 + ((q ^ (lrw & 15)) << 4));
       }
+      // per-row gates: the loads of GB rows together (a row at a time each was
+      // a memory round trip; 256-row tiles have registers for 4); rows past M
+      // read the last row's modulation (their stores are dropped)
+      constexpr int GB = TM == 256 ? 4 : 8;
+      Raw4 graw[EPI == WAM_EPI_BIAS_GATE_RES ? GB : 1];
 #pragma unroll
       for (int k8 = 0; k8 < 8; ++k8) {
         const int ps = b8 * 8 + k8;
         const int row = row_of(r, ps);
+        if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
+          if (k8 % GB == 0 && !gate_held) {
+#pragma unroll
+            for (int k = 0; k < GB; ++k) graw[k] = gate_raw(p, min(m0 + row_u(r, ps + k), p.M - 1), n + p.n_off);
+          }
+        }
         const int off = (row * ld_out + 4 * q) * OB;
         if constexpr (PART) {
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4v, vv[k8]), rout, off, 0, 0);
@@ -622,8 +635,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) gt[e] = row >= gate_split ? gate2[e] : gate[e];
             } else {
-              // rows past M read the last row's modulation (their stores are dropped)
-              ld_mod4(p.gate, p.mod_d, min(m0 + row, p.M - 1), p.gate_index, n + p.n_off, gt);
+              float gb[4];
+              widen4(gtab, p.gate.table_dtype == WAM_F32, gt);
+              widen4(graw[k8 % GB], p.gate.temb_dtype == WAM_F32, gb);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) gt[e] += gb[e];
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[e] = rv[e] + y[e] * gt[e];

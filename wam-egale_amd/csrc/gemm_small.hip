@@ -168,6 +168,11 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
   constexpr bool RES = EPI == WAM_EPI_BIAS_GATE_RES || EPI == WAM_EPI_BIAS_RES;
   Raw4 rraw{};
   if constexpr (RES) rraw = ld4_raw(p.res, p.res_f32 != 0, (int64_t)m * p.ldr + n);
+  Raw4 gtab{}, graw{};
+  if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
+    gtab = ld4_raw(p.gate.table, p.gate.table_dtype == WAM_F32, (int64_t)p.gate_index * p.mod_d + n + p.n_off);
+    graw = gate_raw(p, m, n + p.n_off);
+  }
   const int off[1] = {(m * p.part_ld + c) * 4};
   f32x4 v[1];
   sum_ranges<1>(p, off, v);
@@ -194,8 +199,14 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(LinearParams p) {
     if ((threadIdx.x & 7) == 0) p.oscale[(int64_t)m * (p.seg_n / 32) + n / 32] = (uint8_t)(X + 127);
     return;
   }
-  const float no_gate[4] = {0.f, 0.f, 0.f, 0.f};
-  epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v[0], bv, wsc, no_gate, false, rv);
+  float gate[4] = {0.f, 0.f, 0.f, 0.f}, gb[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
+    widen4(gtab, p.gate.table_dtype == WAM_F32, gate);
+    widen4(graw, p.gate.temb_dtype == WAM_F32, gb);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gate[e] += gb[e];
+  }
+  epi_apply<EPI, W1 ? 1 : 2>(p, out, m, n, v[0], bv, wsc, gate, rv);
 }
 
 int split_reduce(const LinearParams& p, int wb, hipStream_t s) {

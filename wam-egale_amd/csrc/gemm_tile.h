@@ -117,6 +117,37 @@ __device__ inline int lds_off(int r, int c) {
   else return r * 64 + ((c ^ ((r >> 2) & 3)) << 4);
 }
 
+__device__ inline void widen4_bf16(u32x2 t, float out[4]) {
+  out[0] = __uint_as_float(t[0] << 16);
+  out[1] = __uint_as_float(t[0] & 0xffff0000u);
+  out[2] = __uint_as_float(t[1] << 16);
+  out[3] = __uint_as_float(t[1] & 0xffff0000u);
+}
+
+// 4 consecutive values of a bf16 or fp32 vector in two unconditional 8-byte
+// loads (for bf16 the second repeats the first), so that none sits in a
+// branch; widen4 makes fp32 values of them.
+struct Raw4 {
+  u32x2 a, b;
+};
+__device__ inline Raw4 ld4_raw(const void* p, bool f32, int64_t off) {
+  const char* base = static_cast<const char*>(p) + off * (f32 ? 4 : 2);
+  return Raw4{*reinterpret_cast<const u32x2*>(base), *reinterpret_cast<const u32x2*>(base + (f32 ? 8 : 0))};
+}
+__device__ inline void widen4(const Raw4& r, bool f32, float out[4]) {
+  float h[4];
+  widen4_bf16(r.a, h);
+  out[0] = f32 ? __uint_as_float(r.a[0]) : h[0];
+  out[1] = f32 ? __uint_as_float(r.a[1]) : h[1];
+  out[2] = f32 ? __uint_as_float(r.b[0]) : h[2];
+  out[3] = f32 ? __uint_as_float(r.b[1]) : h[3];
+}
+
+// The temb part of the gate of token row m, columns n .. n + 3.
+__device__ inline Raw4 gate_raw(const LinearParams& p, int m, int n) {
+  return ld4_raw(p.gate.temb, p.gate.temb_dtype == WAM_F32, temb_off(p.gate, temb_row(p.gate, m), p.gate_index, p.mod_d, n));
+}
+
 __device__ inline void ld_mod4(const wam_modulation m, int D, int64_t row, int idx,
                                int d, float out[4]) {
   const int64_t toff = temb_off(m, temb_row(m, row), idx, D, d);
@@ -202,7 +233,7 @@ __device__ __forceinline__ void fetch_frags(const char* abase, const char* bbase
 template <int EPI, int WB>
 __device__ __forceinline__ void epi_apply(const LinearParams& p, void* out, int m, int n, const f32x4 v,
                                           const float (&bv)[4], const float (&wsc)[4],
-                                          const float (&gate_pre)[4], bool gate_held, const float (&rv)[4]) {
+                                          const float (&gate)[4], const float (&rv)[4]) {
   float y[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) y[e] = WB == 1 ? v[e] * wsc[e] + bv[e] : v[e] + bv[e];
@@ -211,15 +242,8 @@ __device__ __forceinline__ void epi_apply(const LinearParams& p, void* out, int 
     for (int e = 0; e < 4; ++e) y[e] = gelu_tanh(y[e]);
   } else if constexpr (EPI == WAM_EPI_BIAS_GATE_RES || EPI == WAM_EPI_BIAS_RES) {
     if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
-      float gt[4];
-      if (gate_held) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) gt[e] = gate_pre[e];
-      } else {
-        ld_mod4(p.gate, p.mod_d, m, p.gate_index, n + p.n_off, gt);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = rv[e] + y[e] * gt[e];
+      for (int e = 0; e < 4; ++e) y[e] = rv[e] + y[e] * gate[e];
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = rv[e] + y[e];
@@ -467,8 +491,13 @@ __global__ __launch_bounds__(C::kThreads, C::BLOCKS) void gemm_bf16_kernel(Linea
   // loop, which has no registers to spare for it) when the tile's rows read
   // at most two consecutive modulation rows (one or two samples, or latent
   // frames): gate for the rows before gate_split, gate2 from there on.  Rows
-  // that read more (one modulation row per token) load theirs per row.
+  // that read more (one modulation row per token) load theirs per row, those
+  // of kGateBatch iterations together (a row at a time each was a memory round
+  // trip: 2325 x 3072 x 3072, one modulation row per token, 70 -> 64 us; the
+  // four-wave kernel's fp8 2325 x 14336 x 3072 134 -> 120).
   float gate[4] = {0.f, 0.f, 0.f, 0.f}, gate2[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kGateBatch = 4;
+  Raw4 gtab{};
   bool gate_held = false;
   int gate_split = 0;  // first tile row served by the second modulation row
   if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
@@ -481,6 +510,7 @@ __global__ __launch_bounds__(C::kThreads, C::BLOCKS) void gemm_bf16_kernel(Linea
     const int nc = min(n, p.seg_n - 4) + p.n_off;
     ld_mod4(p.gate, p.mod_d, m0, p.gate_index, nc, gate);
     ld_mod4(p.gate, p.mod_d, m_last, p.gate_index, nc, gate2);
+    gtab = ld4_raw(p.gate.table, p.gate.table_dtype == WAM_F32, (int64_t)p.gate_index * p.mod_d + nc);
   }
   // q-norm epilogue (no RoPE here): the gamma of the lane's 4 columns and the
   // segment's sums-of-squares array.  With 256-column tiles a wave holds one
@@ -524,11 +554,19 @@ __global__ __launch_bounds__(C::kThreads, C::BLOCKS) void gemm_bf16_kernel(Linea
     // the round's residual rows have landed (one wait per round, which also
     // drains the previous round's stores)
     if constexpr (RES) wait_vmcnt<0>();
+    Raw4 graw[kGateBatch];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const int rr = (it * C::kWaves + wave) * RPI + lane / QPR;  // row within the round
       const int row = rd * ROUND + rr;
       const int m = m0 + row;
+      if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
+        if (it % kGateBatch == 0 && !gate_held) {
+#pragma unroll
+          for (int k = 0; k < kGateBatch; ++k)
+            graw[k] = gate_raw(p, min(m + k * C::kWaves * RPI, p.M - 1), min(n, p.seg_n - 4) + p.n_off);
+        }
+      }
       if constexpr (NORM) {
         // y = bf16(acc + b) as the bias epilogue rounds it; the row's sum of
         // y^2 over the tile's 256 columns (every lane of the wave takes part
@@ -575,7 +613,16 @@ __global__ __launch_bounds__(C::kThreads, C::BLOCKS) void gemm_bf16_kernel(Linea
         float gsel[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) gsel[e] = row >= gate_split ? gate2[e] : gate[e];
-        epi_apply<EPI, C::WB>(p, out, m, n, v, bv, wsc, gsel, gate_held, rv);
+        if constexpr (EPI == WAM_EPI_BIAS_GATE_RES) {
+          if (!gate_held) {
+            float gb[4];
+            widen4(gtab, p.gate.table_dtype == WAM_F32, gsel);
+            widen4(graw[it % kGateBatch], p.gate.temb_dtype == WAM_F32, gb);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gsel[e] += gb[e];
+          }
+        }
+        epi_apply<EPI, C::WB>(p, out, m, n, v, bv, wsc, gsel, rv);
       }
     }
     if (rd + 1 < NROUNDS) {
@@ -618,32 +665,6 @@ __device__ inline void sum_ranges(const LinearParams& p, const int (&off)[NCH], 
   for (int c = 0; c < NCH; ++c) v[c] = f32x4{};
   if (p.k_split <= 4) return add_ranges<4, NCH>(p, 0, off, v);
   for (int r0 = 0; r0 < p.k_split; r0 += 8) add_ranges<8, NCH>(p, r0, off, v);
-}
-
-__device__ inline void widen4_bf16(u32x2 t, float out[4]) {
-  out[0] = __uint_as_float(t[0] << 16);
-  out[1] = __uint_as_float(t[0] & 0xffff0000u);
-  out[2] = __uint_as_float(t[1] << 16);
-  out[3] = __uint_as_float(t[1] & 0xffff0000u);
-}
-
-// 4 consecutive values of a bf16 or fp32 vector in two unconditional 8-byte
-// loads (for bf16 the second repeats the first), so that none sits in a
-// branch; widen4 makes fp32 values of them.
-struct Raw4 {
-  u32x2 a, b;
-};
-__device__ inline Raw4 ld4_raw(const void* p, bool f32, int64_t off) {
-  const char* base = static_cast<const char*>(p) + off * (f32 ? 4 : 2);
-  return Raw4{*reinterpret_cast<const u32x2*>(base), *reinterpret_cast<const u32x2*>(base + (f32 ? 8 : 0))};
-}
-__device__ inline void widen4(const Raw4& r, bool f32, float out[4]) {
-  float h[4];
-  widen4_bf16(r.a, h);
-  out[0] = f32 ? __uint_as_float(r.a[0]) : h[0];
-  out[1] = f32 ? __uint_as_float(r.a[1]) : h[1];
-  out[2] = f32 ? __uint_as_float(r.b[0]) : h[2];
-  out[3] = f32 ? __uint_as_float(r.b[1]) : h[3];
 }
 
 }  // namespace wam
