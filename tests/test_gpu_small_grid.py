@@ -22,13 +22,14 @@ def _ulp(ref):
     return 2.0 ** -8 * ref.abs().max().item() + 2e-3
 
 
-# Rows at the edges of the 32, 64, 128, 192, 224 and 256 row tiles, one k-tile
+# Rows at the edges of the tiles (32 to 256 rows, 128 or 256 columns), one k-tile
 # and an uneven number of them (65 over 10 or more ranges), partial column
 # tiles, three segments split over k (action tokens) and whole.
 SHAPES = [(1, 64, 128, 1), (1, 4160, 3072, 1), (32, 3072, 3072, 3), (33, 3072, 3072, 1), (64, 4160, 1536, 1),
           (65, 3072, 3072, 1), (129, 14336, 3072, 1), (193, 3072, 3072, 1), (225, 8960, 1536, 1),
           (400, 3072, 3072, 3), (780, 4160, 3072, 1), (1024, 8960, 1536, 1), (1560, 4160, 3072, 1),
-          (2325, 14336, 3072, 1), (40, 3072, 192, 1), (300, 3072, 200, 1), (512, 3072, 3072, 2)]
+          (2325, 14336, 3072, 1), (2325, 3072, 3072, 1), (1000, 1536, 8960, 1), (1300, 14336, 3072, 1),
+          (1921, 3072, 3072, 1), (3001, 3072, 3072, 1), (40, 3072, 192, 1), (300, 3072, 200, 1), (512, 3072, 3072, 2)]
 
 
 @pytest.mark.parametrize("M,K,N,nseg", SHAPES)
@@ -47,7 +48,7 @@ def test_bias_and_gelu(dev, M, K, N, nseg):
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 4160, 3072), (33, 3072, 3072), (224, 14336, 3072), (400, 4160, 3072),
-                                   (780, 14336, 3072), (300, 3072, 200)])
+                                   (780, 14336, 3072), (300, 3072, 200), (2325, 3072, 3072), (3001, 3072, 3072)])
 @pytest.mark.parametrize("fp32", [False, True])
 def test_residuals(dev, M, K, N, fp32):
     from wam_ops import ops

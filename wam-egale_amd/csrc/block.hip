@@ -36,6 +36,7 @@ int rms_rope(const wam_rms_rope_args*, const wam_kv_layout_args*, hipStream_t);
 int attention(const wam_attention_args*, hipStream_t);
 int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys);
 int64_t linear_workspace_bytes(int M, int seg_n, int n_seg, int K);
+int64_t linear_partials_bytes(int M, int seg_n, int n_seg, int K);
 int64_t linear_f8mm_bytes(int M, int N, int K);
 bool linear_norm_in_epilogue(int M, int seg_n, int n_seg, int K, int64_t ws_bytes, bool rope);
 int kv_layout(const wam_kv_layout_args*, hipStream_t);
@@ -110,9 +111,10 @@ static Layout layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
   // One region: the kernels that use it run one after another on the stream.
   const int64_t need[] = {attention_workspace_bytes(B, M, D / 128, (int64_t)M + (pool > 0 ? pool : 0)),
                           attention_workspace_bytes(B, M, D / 128, Lc),
-                          linear_workspace_bytes((int)R, D, 3, D),   // QKV
+                          linear_workspace_bytes((int)R, D, 3, D), linear_partials_bytes((int)R, D, 3, D),  // QKV
                           linear_workspace_bytes(Bc * Lc, D, 2, D),  // cross K/V
-                          linear_workspace_bytes((int)R, D, 1, D),   // self_out, cross_q, cross_out
+                          // self_out, cross_q, cross_out
+                          linear_workspace_bytes((int)R, D, 1, D), linear_partials_bytes((int)R, D, 1, D),
                           linear_workspace_bytes((int)R, F, 1, D),   // FFN1
                           linear_workspace_bytes((int)R, D, 1, F),   // FFN2
                           linear_f8mm_bytes((int)R, F, D), linear_f8mm_bytes((int)R, D, F)};  // both with fp8 activations

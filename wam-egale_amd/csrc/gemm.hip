@@ -31,28 +31,22 @@ namespace wam {
 // texture unit's address and command queues, and a wave that cannot issue a
 // load cannot issue the MFMAs behind it either (4680x3072x14336:
 // SQ_VMEM_TA_ADDR_FIFO_FULL 1.7e7 -> 4.5e5 cycles, k loop 369 -> 337 us).
-struct CfgW4 {
-  static constexpr int BM = 256, BN = 256, BK = 64, WB = 2, kThreads = 256;
+template <int TM, int WB_>
+struct CfgW4Rows {
+  static constexpr int BM = TM, BN = 256, BK = 64, WB = WB_, kThreads = 256;
   static constexpr bool kW4 = true;
 };
+using CfgW4 = CfgW4Rows<256, 2>;
 // The same kernel on 224 x 256 tiles, the four waves side by side along n
 // (224 x 64 each, 7 x 2 MFMA blocks): 4680 rows are 21 such tiles (0.5% of
 // padding against 3.9% for 19 x 256), and a 3072-column GEMM then fills 252
-// of the 256 CUs in one round of 7/8 of a 256-row tile's work.
-struct CfgW4t224 {
-  static constexpr int BM = 224, BN = 256, BK = 64, WB = 2, kThreads = 256;
-  static constexpr bool kW4 = true;
-};
+// of the 256 CUs in one round of 7/8 of a 256-row tile's work.  And so on
+// down to 128 rows (4 x 2 blocks) where a shorter tile fills a round better.
+using CfgW4t224 = CfgW4Rows<224, 2>;
 // The same two tilings with fp8 e4m3 weights (widened to bf16 on the way
 // into LDS; per-column scales in the epilogue).
-struct CfgW4f8 {
-  static constexpr int BM = 256, BN = 256, BK = 64, WB = 1, kThreads = 256;
-  static constexpr bool kW4 = true;
-};
-struct CfgW4t224f8 {
-  static constexpr int BM = 224, BN = 256, BK = 64, WB = 1, kThreads = 256;
-  static constexpr bool kW4 = true;
-};
+using CfgW4f8 = CfgW4Rows<256, 1>;
+using CfgW4t224f8 = CfgW4Rows<224, 1>;
 
 // The NM MFMAs of one 16-deep sub-step with the NR fragment reads of the
 // next sub-step, W LDS writes and V global loads spread evenly between them
@@ -79,7 +73,7 @@ __device__ __forceinline__ void w4_sched() {
 // RF32 / OF32: the residual / output is fp32 (else bf16; OF32 = 2: e4m3 with
 // e8m0 exponents per 32 columns, the MX output); compile-time so
 // that the epilogue's loads and stores are branch-free.  TM: tile rows, 256
-// (waves 2 x 2, 128 x 128 each) or 224 (waves 1 x 4, 224 x 64 each).
+// (waves 2 x 2, 128 x 128 each) or 128 to 224 (waves 1 x 4, TM x 64 each).
 // WB: bytes per weight element, 2 (bf16) or 1 (fp8 e4m3 with per-column
 // fp32 scales).  fp8 weight rows are 64 bytes per k-step: a thread loads 16
 // of them (a quarter row) and widens them exactly to bf16 in registers as it
@@ -93,10 +87,10 @@ __device__ __forceinline__ void w4_sched() {
 // 32 k instead of a row scale, applied as the MFMA's block scales.
 template <int EPI, int RF32, int OF32, int TM, int WB = 2, bool F8MM = false, bool AMX = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
-  static_assert(TM == 256 || TM == 224 || (TM == 128 && F8MM), "tile rows");
+  static_assert(TM == 256 || TM == 224 || ((TM == 128 || TM == 160 || TM == 192) && WB == 2), "tile rows");
   static_assert(WB == 2 || WB == 1, "weight bytes");
   constexpr bool MXO = OF32 == 2;  // e4m3 output with e8m0 exponents per 32 columns
-  static_assert(!F8MM || (WB == 2 && TM != 256), "fp8 MFMA: 224- or 128-row tiles");
+  static_assert(!F8MM || (WB == 2 && TM != 256), "fp8 MFMA: up to 224-row tiles");
   static_assert(!F8MM || AMX || EPI == WAM_EPI_BIAS || EPI == WAM_EPI_BIAS_GELU || EPI == kEpiPartial,
                 "fp8 MFMA with per-row activation scales: bias or GELU epilogue");
   static_assert(!AMX || (F8MM && !MXO && EPI != WAM_EPI_BIAS_GELU), "MX activations: fp8 MFMA, bf16 output");
@@ -196,7 +190,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
     return n;
   };
   // The staging sets go to LDS and are reloaded in three parts over a k-step.
-  constexpr int P1 = WB == 1 ? 5 : (NL == 16 ? 6 : 5), P2 = WB == 1 ? 9 : (NL == 16 ? 11 : 10);
+  constexpr int P1 = WB == 1 ? 5 : (NL + 2) / 3, P2 = WB == 1 ? 9 : (2 * NL + 2) / 3;
   using I0 = std::integral_constant<int, 0>;
   using IP1 = std::integral_constant<int, P1>;
   using IP2 = std::integral_constant<int, P2>;
@@ -462,8 +456,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
   typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
   typedef unsigned int u32x2v __attribute__((ext_vector_type(2)));
   // Tile row handled by pass ps (0..31) of round r: rows 64 r .. +64 of each
-  // wave row (TM = 256), or rows 128 r .. +128 (TM = 224, whose second round
-  // has 96 rows, passes 0..23).
+  // wave row (TM = 256), or rows 128 r .. +128 (the others, whose second round
+  // has TM - 128 rows: 96, passes 0..23, with 224).
   auto row_of = [&](int r, int ps) {
     const int rr = ps * 4 + (tid >> 6);
     return TM == 256 ? (rr >> 6) * 128 + 64 * r + (rr & 63) : 128 * r + rr;
@@ -496,7 +490,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
   auto round = [&](auto r_c, auto nrm_c, auto rope_c) {
     constexpr int r = decltype(r_c)::value;
     constexpr bool NRM = decltype(nrm_c)::value, ROPE = decltype(rope_c)::value;
-    constexpr int nps = (TM == 224 && r == 1) ? 24 : 32;
+    constexpr int nps = TM == 256 || r == 0 ? 32 : (TM - 128) / 4;
     u32x4v rraw[RES ? 32 : 1];
     if constexpr (RES) {
 #pragma unroll
@@ -544,8 +538,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(LinearParams p) {
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     // The wave's m-blocks of this round, as 1 KB fp32 rows: TM = 256, blocks
-    // 2r and 2r+1 into L0 (wave row 0) or L1 (wave row 1); TM = 224, blocks
-    // 4r .. 4r+3 (of 7), two into each buffer.
+    // 2r and 2r+1 into L0 (wave row 0) or L1 (wave row 1); the others, blocks
+    // 4r .. 4r+3 (of TM / 32), two into each buffer.
 #pragma unroll
     for (int ii = 0; ii < (TM == 256 ? 2 : 4); ++ii) {
       const int i = TM == 256 ? 2 * r + ii : 4 * r + ii;
@@ -843,7 +837,7 @@ static int launch_gemm(LinearParams& p, hipStream_t s) {
   }
   switch (p.epi) {
     case kEpiBiasNorm:
-      if constexpr (C::kW4 || std::is_same_v<C, Cfg320x256w8>) {
+      if constexpr ((C::kW4 && C::BM >= 224) || std::is_same_v<C, Cfg320x256w8>) {
         WAM_REQUIRE(C::kW4 || p.nfreq == nullptr, "wam_linear: the 320-row q-norm epilogue has no RoPE");
         launch_tiles<C, kEpiBiasNorm>(dim3(grid), p, s);
       } else {
@@ -945,7 +939,13 @@ static int launch_big(LinearParams& p, int64_t ws_bytes, hipStream_t s) {
 
 int w4_tiles(LinearParams& p, int tm, int wb, hipStream_t s) {
   if (wb == 1) return tm == 224 ? launch_gemm<CfgW4t224f8>(p, s) : launch_gemm<CfgW4f8>(p, s);
-  return tm == 224 ? launch_gemm<CfgW4t224>(p, s) : launch_gemm<CfgW4>(p, s);
+  switch (tm) {
+    case 128: return launch_gemm<CfgW4Rows<128, 2>>(p, s);
+    case 160: return launch_gemm<CfgW4Rows<160, 2>>(p, s);
+    case 192: return launch_gemm<CfgW4Rows<192, 2>>(p, s);
+    case 224: return launch_gemm<CfgW4t224>(p, s);
+    default: return launch_gemm<CfgW4>(p, s);
+  }
 }
 
 // Cost of a launch in 256x256-tile times: the 256-row plan (whole rounds,
@@ -1012,7 +1012,7 @@ static SplitPlan f8mm_plan(int M, int N, int K, int64_t ws_bytes) {
       const int64_t rounds = (n * ks + cus - 1) / cus, steps = (nk + ks - 1) / ks;
       const double used = n * ks < cus ? (double)(n * ks) / cus : 1.0;
       double cost = kSmallLaunch + (double)rounds * (t.round + (double)steps * (t.step + t.share * used));
-      if (ks > 1) cost += split_reduce_us(ks * plane);
+      if (ks > 1) cost += split_reduce_us(ks * plane, false);
       if (cost < best_cost - 1e-9) best_cost = cost, best = SplitPlan{t.tm, (int)ks};
     }
   }
@@ -1026,6 +1026,12 @@ int64_t linear_workspace_bytes(int M, int seg_n, int n_seg, int K) {
     return K % 64 == 0 ? split_plan_bytes(split_plan(M, seg_n, n_seg, K, 2, INT64_MAX), M, seg_n, n_seg) : 0;
   }
   return plan_workspace(gemm_plan(M, seg_n, n_seg, K, device_cu_count(), INT64_MAX), M, seg_n);
+}
+
+// What linear_partials can use.
+int64_t linear_partials_bytes(int M, int seg_n, int n_seg, int K) {
+  if (K % 64 != 0 || uses_big_tiles(M, seg_n, n_seg)) return 0;
+  return split_plan_bytes(split_plan(M, seg_n, n_seg, K, 2, INT64_MAX, true), M, seg_n, n_seg);
 }
 
 // What a launch with fp8 activations can use.
@@ -1167,7 +1173,7 @@ int linear_partials(const wam_linear_args* a, hipStream_t s, LinearParams* p, bo
   *split = false;
   WAM_TRY(linear_setup(a, *p));
   if (a->w_dtype != WAM_BF16 || a->a_dtype != WAM_BF16 || uses_big_tiles(a->M, a->seg_n, a->n_seg)) return WAM_OK;
-  const SplitPlan g = split_plan(a->M, a->seg_n, a->n_seg, a->K, 2, a->workspace ? a->workspace_bytes : 0);
+  const SplitPlan g = split_plan(a->M, a->seg_n, a->n_seg, a->K, 2, a->workspace ? a->workspace_bytes : 0, true);
   if (g.ks == 1) return WAM_OK;
   *split = true;
   return split_tiles(*p, g, 2, s);

@@ -41,14 +41,15 @@ struct LinearParams {
   uint8_t* oscale;
 };
 
-// Cost of a launch and of the reduce pass over `bytes` of partial sums, us.
+// Cost of a launch, and of reducing `bytes` of partial sums in a pass of its
+// own or in a row pass that runs anyway, us.
 constexpr double kSmallLaunch = 2.6;
-inline double split_reduce_us(int64_t bytes) { return 4.1 + 0.28e-6 * (double)bytes; }
+inline double split_reduce_us(int64_t bytes, bool fused) { return (fused ? 0.0 : 4.1) + 0.28e-6 * (double)bytes; }
 // Tile (an index into the small-grid plan's table) and k ranges of a launch.
 struct SplitPlan {
   int tile, ks;
 };
-SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_bytes);
+SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_bytes, bool fused = false);
 int64_t split_plan_bytes(const SplitPlan& g, int M, int seg_n, int n_seg);
 int split_tiles(LinearParams& p, const SplitPlan& g, int wb, hipStream_t s);
 int split_reduce(const LinearParams& p, int wb, hipStream_t s);
@@ -58,8 +59,8 @@ int split_reduce(const LinearParams& p, int wb, hipStream_t s);
 int linear_partials(const wam_linear_args* a, hipStream_t s, LinearParams* p, bool* split);
 int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s);
 int split_ln(const LinearParams& p, const wam_ln_args& l, hipStream_t s);
-// One launch of the four-wave kernel on 224- or 256-row tiles (bf16 or fp8
-// weights); with p.k_split > 1 its partial sums only.
+// One launch of the four-wave kernel on tm-row tiles (128 to 256; fp8 weights
+// 224 or 256); with p.k_split > 1 its partial sums only.
 int w4_tiles(LinearParams& p, int tm, int wb, hipStream_t s);
 
 constexpr int kEpiPartial = 100;   // kernel epilogue of a split-K range: raw fp32 sums
