@@ -115,6 +115,24 @@ def test_rows_linear(dev, R, N, K, dtypes):
         assert err <= bound, (act_in, act_out, err, bound)
 
 
+# bf16 rows on the matrix cores: partial blocks of 32 rows and outputs, fewer
+# k-steps of 16 than waves, a share of k that is no multiple of the loads made
+# together; 7 and 8 rows on either side of the dispatch at 16416 outputs.
+@pytest.mark.parametrize("R,N,K", [(1, 1, 16), (28, 18432, 3072), (33, 40, 208), (7, 16416, 64), (8, 16416, 64), (64, 31, 1552)])
+@pytest.mark.parametrize("od", [torch.float32, torch.bfloat16])
+def test_rows_linear_bf16(dev, R, N, K, od):
+    from wam_ops import ops
+    x, w, b = _randn((R, K), 1, 1.0, torch.bfloat16), _randn((N, K), 2, 0.02, torch.bfloat16), _randn((N,), 3, 0.02)
+    scale = (x.double().abs() @ w.double().abs().t()).max().item() + 1e-3
+    for act_in, act_out in ((None, None), ("silu", None), (None, "silu")):
+        y = ops.rows_linear(x.to(dev), w.to(dev), b.to(dev), act_in=act_in, act_out=act_out, out_dtype=od)
+        ref = _rows_ref(x, w, b, act_in, act_out, torch.bfloat16, od)
+        err = (y.cpu().double() - ref).abs().max().item()
+        # fp32 sums; SiLU's fp32 form may round an input the other way (2^-8 of it); the output's rounding
+        bound = (1e-5 + (2 ** -8 if act_in else 0)) * scale + (2 ** -7 * ref.abs().max().item() if od == torch.bfloat16 else 0.0)
+        assert err <= bound, (act_in, act_out, err, bound)
+
+
 def test_head_norm(dev):
     from wam_ops import ops
     B, M, D, Fr = 2, 60, 256, 3

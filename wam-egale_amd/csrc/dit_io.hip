@@ -257,6 +257,64 @@ __global__ __launch_bounds__(512) void rows_linear_act_kernel(wam_rows_linear_ar
   if (nc > 0) rl_store(a, acc, lane, n0, r0, nr, nc);
 }
 
+// bf16 x and weights: 32 rows x 32 outputs a workgroup on the matrix cores,
+// its 8 waves a share of k each, their sums added in wave order.  The dot
+// products above pass over the weights once per 8 rows and spend R x N x K
+// lane operations; this kernel is bound by the fragment loads (32 bytes of a
+// row's 128-byte line at a time; with a second set of loads in flight it was
+// slower).  us, weights cold, with SiLU: 28 x 18432 x 3072 129 -> 61, 224 x
+// 18432 x 3072 811 -> 248, 28 x 9216 x 1536 40 -> 22, 224 x 30 x 3072 18 -> 13.
+template <bool ACT>
+__global__ __launch_bounds__(512) void rows_linear_mfma_kernel(wam_rows_linear_args a) {
+  constexpr int U = 8, LD = 36;  // k-steps loaded together; padded row of the exchange
+  __shared__ __attribute__((aligned(16))) float red[8][32][LD];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+  const int steps = a.K / 16, s0 = steps * wave / 8, s1 = steps * (wave + 1) / 8;
+  // rows and outputs past the end repeat the last ones and are not stored
+  const bf16* w = static_cast<const bf16*>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.ldw + 8 * half;
+  const bf16* x = static_cast<const bf16*>(a.x) + (int64_t)min(r0 + l32, a.R - 1) * a.ldx + 8 * half;
+  f32x16 acc{};
+  for (int s = s0; s < s1; s += U) {
+    bf16x8 fw[U], fx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(s + u, s1 - 1) * 16;
+      fw[u] = ld_bf16x8(w + k);
+      fx[u] = ld_bf16x8(x + k);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s + u >= s1) break;
+      if constexpr (ACT) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) fx[u][e] = static_cast<bf16>(silu_fast(static_cast<float>(fx[u][e])));
+      }
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[u], fx[u], acc, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *reinterpret_cast<float4*>(&red[wave][l32][8 * g + 4 * half]) =
+        make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+  __syncthreads();
+  const int r = tid >> 4;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = 2 * (tid & 15) + i, n = n0 + c;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v += red[q][r][c];
+    if (r0 + r >= a.R || n >= a.N) continue;
+    if (a.bias) v += ld_scalar(a.bias, a.bias_dtype, n);
+    if (a.act_out == WAM_ACT_SILU) v = silu(round_to(v, a.out_dtype));
+    const int64_t o = (int64_t)(r0 + r) * a.ldo + n;
+    if (a.out_dtype == WAM_F32) static_cast<float*>(a.out)[o] = v;
+    else static_cast<bf16*>(a.out)[o] = static_cast<bf16>(v);
+  }
+}
+
 static bool fd(int d) { return d == WAM_F32 || d == WAM_BF16; }
 
 int rows_linear(const wam_rows_linear_args* a, hipStream_t s) {
@@ -274,6 +332,18 @@ int rows_linear(const wam_rows_linear_args* a, hipStream_t s) {
   const auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool vec = a->K % 8 == 0 && a->ldx % 8 == 0 && a->ldw % 8 == 0 && al(a->x) && al(a->w);
   const bool act = a->act_in != WAM_ACT_NONE;
+  // Fewer than 8 rows take it where two workgroups per CU cover the outputs (1
+  // x 9216 x 1536 15.9 -> 13.8 us); beyond, the dot products' whole-row loads
+  // are the faster way through the weights (1 x 18432 x 3072 31 us against 45).
+  const int blocks = (a->N - 1) / 32 + 1;
+  if (vec && a->K % 16 == 0 && a->x_dtype == WAM_BF16 && a->w_dtype == WAM_BF16 &&
+      (a->R >= 8 || blocks <= 2 * device_cu_count())) {
+    const dim3 grid((unsigned)blocks, (unsigned)((a->R - 1) / 32 + 1));
+    if (act) hipLaunchKernelGGL(rows_linear_mfma_kernel<true>, grid, dim3(512), 0, s, *a);
+    else hipLaunchKernelGGL(rows_linear_mfma_kernel<false>, grid, dim3(512), 0, s, *a);
+    WAM_LAUNCHED("rows_linear_mfma_kernel");
+    return WAM_OK;
+  }
   const int per_wg = kRlOut * (act ? 8 : 4);
   const dim3 grid((unsigned)((a->N + per_wg - 1) / per_wg), (unsigned)((a->R + kRlRows - 1) / kRlRows));
   if (act) {
