@@ -74,3 +74,20 @@ def test_block_of_few_rows(dev, dim, ffn, B, grid, temb_len, norm2):
                  "residual1", "norm2", "cross_q_linear", "cross_q", "residual2", "modulated3"):
         want = keep[name].reshape(-1, keep[name].shape[-1]) if keep[name].dim() == 3 else keep[name].flatten(2).reshape(-1, dim)
         assert_close(dbg[name].cpu().float(), want, 2.0 ** -7 * want.abs().max().item() + 4e-3, 0.9999, f"{name} {dim} {B}x{M}")
+
+
+def test_rope_table_batch_is_refused(dev, monkeypatch):
+    """A table of neither one nor B samples, past the binding's own check: the
+    row pass over partial sums refuses it as the one over rows does."""
+    from wam_ops import native, synthetic
+    from wam_ops.block import TransformerBlock
+    shape = synthetic.BlockShape(256, 2, 512)
+    with torch.device("meta"):
+        blk = TransformerBlock(256, 512, 2, cross_attn_norm=True)
+    blk.load_state_dict(synthetic.block_params(shape, seed=3, device=dev), assign=True)
+    monkeypatch.setattr(native, "_check", lambda *a: None)
+    for M in (16, 3000):
+        x, ctx, temb, freqs = synthetic.block_inputs(shape, 2, M, (1, 1, M), context_len=20, context_batch=2, seed=4, device=dev)
+        with torch.no_grad(), pytest.raises(RuntimeError, match="freq batch"):
+            blk(x, ctx, temb, freqs[:1].expand(3, *freqs.shape[1:]))
+    torch.cuda.synchronize()

@@ -389,9 +389,7 @@ static void launch_rms_rope(const wam_rms_rope_args& a, const wam_kv_layout_args
   else hipLaunchKernelGGL((rms_rope_kernel<CH, false>), grid, block, 0, s, a, wam_kv_layout_args{});
 }
 
-// kv (may be null): the KV pool's bookkeeping, done by one workgroup of the
-// launch (pools of up to kLayoutSlots * 256 slots).
-int rms_rope(const wam_rms_rope_args* a, const wam_kv_layout_args* kv, hipStream_t s) {
+int rms_rope_check(const wam_rms_rope_args* a) {
   WAM_REQUIRE(a != nullptr, "wam_rms_rope: null args");
   WAM_REQUIRE(a->n_tensors == 1 || a->n_tensors == 2, "wam_rms_rope: n_tensors must be 1 or 2");
   WAM_REQUIRE(a->D > 0 && a->D % 8 == 0 && a->D <= 4096, "wam_rms_rope: D=%d unsupported", a->D);
@@ -406,6 +404,13 @@ int rms_rope(const wam_rms_rope_args* a, const wam_kv_layout_args* kv, hipStream
                 (a->freq_batch == 1 || a->freq_batch == a->rows / a->tokens),
                 "wam_rms_rope: freq batch %d / tokens %d contract", a->freq_batch, a->tokens);
   }
+  return WAM_OK;
+}
+
+// kv (may be null): the KV pool's bookkeeping, done by one workgroup of the
+// launch (pools of up to kLayoutSlots * 256 slots).
+int rms_rope(const wam_rms_rope_args* a, const wam_kv_layout_args* kv, hipStream_t s) {
+  WAM_TRY(rms_rope_check(a));
   if (a->rows == 0) return WAM_OK;
   const int ch = (a->D / 8 + 63) / 64;
   if (ch <= 1) launch_rms_rope<1>(*a, kv, s);

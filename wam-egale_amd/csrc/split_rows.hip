@@ -222,7 +222,10 @@ static void launch_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, c
   else hipLaunchKernelGGL((split_rms_rope_kernel<NCH, false>), grid, block, 0, s, p, r, wam_kv_layout_args{});
 }
 
+int rms_rope_check(const wam_rms_rope_args*);
+
 int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s) {
+  WAM_TRY(rms_rope_check(&r));
   switch ((p.seg_n + 1023) / 1024) {
     case 1: launch_rms_rope<1>(p, r, kv, s); break;
     case 2: launch_rms_rope<2>(p, r, kv, s); break;
