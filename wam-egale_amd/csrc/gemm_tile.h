@@ -146,7 +146,8 @@ __device__ inline void widen4(const Raw4& r, bool f32, float out[4]) {
 
 // The temb part of the gate of token row m, columns n .. n + 3.
 __device__ inline Raw4 gate_raw(const LinearParams& p, int m, int n) {
-  return ld4_raw(p.gate.temb, p.gate.temb_dtype == WAM_F32, temb_off(p.gate, temb_row(p.gate, m), p.gate_index, p.mod_d, n));
+  const int64_t trow = p.gate.temb_len == p.gate.tokens ? m : temb_row(p.gate, m);
+  return ld4_raw(p.gate.temb, p.gate.temb_dtype == WAM_F32, temb_off(p.gate, trow, p.gate_index, p.mod_d, n));
 }
 
 __device__ inline void ld_mod4(const wam_modulation m, int D, int64_t row, int idx,

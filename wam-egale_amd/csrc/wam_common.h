@@ -246,10 +246,10 @@ __device__ inline void ld8_f32(const void* p, int dtype, int64_t off, float out[
 // Row of temb that serves token row `row`: per sample, per token, or per
 // group of tokens / temb_len consecutive tokens (one latent frame).
 __device__ inline int64_t temb_row(const wam_modulation& m, int64_t row) {
-  if (m.temb_len == m.tokens) return row;
   int64_t b, t;
   split_row(row, m.tokens, b, t);
   if (m.temb_len == 1) return b;
+  if (m.temb_len == m.tokens) return b * m.tokens + t;
   const uint32_t group = (uint32_t)m.tokens / (uint32_t)m.temb_len;
   return b * m.temb_len + (uint32_t)t / group;
 }
