@@ -132,10 +132,11 @@ typedef struct {
    * no fp8 path. */
   int w_dtype;
   const float* w_scale[3];
-  /* Optional workspace for the split-K tail: when the 256x256 tiles leave
-   * a partial last round, the remaining output columns may run split over k
-   * with fp32 partial sums here (at least wam_linear_workspace_bytes(M,
-   * seg_n, n_seg, K) bytes), or, without it, as smaller tiles.  Not in the
+  /* Optional workspace for fp32 partial sums of k ranges, where a grid of
+   * few tiles, or the columns left over by a partial last round of 256x256
+   * tiles, run split over k: wam_linear_workspace_bytes(M, seg_n, n_seg, K)
+   * bytes hold the plan for bf16 operands (fp8 ones plan within what is
+   * there); with less, fewer ranges, and with none whole k.  Not in the
    * reference (cuBLASLt picks its own algorithm and workspace). */
   void* workspace; int64_t workspace_bytes;
   /* Optional q/k-norm epilogue (WAM_EPI_BIAS only): the across-heads RMSNorm
@@ -252,8 +253,8 @@ typedef struct {
   const void* k; const void* v; int64_t kv_bstride, kv_rstride; int Mk;
   const int64_t* kv_rows; int kv_batch;
   float scale;
-  /* Optional workspace for key-range splits of the last dispatch round
-   * (used when the query grid alone would leave CUs idle): at least
+  /* Optional workspace for key-range splits (used when the query grid alone
+   * would leave CUs idle): at least
    * wam_attention_workspace_bytes(B, Mq, H, max_keys) bytes, or NULL to run
    * unsplit.  max_keys: host-side upper bound of Mk + n_hist (0 = Mk), used
    * only to plan the split.  Not in the reference (its FlashAttention call
