@@ -242,6 +242,6 @@ def test_small_grid_plan_workspace():
             n = h.wam_linear_workspace_bytes(M, N, n_seg, K)
             ks, rest = divmod(n, M * N * n_seg * 4)
             assert rest == 0 and (ks == 0 or 2 <= ks <= min(32, K // 64)), (M, N, n_seg, K, n)
-    assert h.wam_linear_workspace_bytes(32, 3072, 1, 14336) == 10 * 32 * 3072 * 4
+    assert h.wam_linear_workspace_bytes(32, 3072, 1, 14336) == 5 * 32 * 3072 * 4
     assert h.wam_linear_workspace_bytes(224, 3072, 1, 14336) == 5 * 224 * 3072 * 4
     assert h.wam_linear_workspace_bytes(224, 14336, 1, 3072) == 0

@@ -29,7 +29,8 @@ SHAPES = [(1, 64, 128, 1), (1, 4160, 3072, 1), (32, 3072, 3072, 3), (33, 3072, 3
           (65, 3072, 3072, 1), (129, 14336, 3072, 1), (193, 3072, 3072, 1), (225, 8960, 1536, 1),
           (400, 3072, 3072, 3), (780, 4160, 3072, 1), (1024, 8960, 1536, 1), (1560, 4160, 3072, 1),
           (2325, 14336, 3072, 1), (2325, 3072, 3072, 1), (1000, 1536, 8960, 1), (1300, 14336, 3072, 1),
-          (1921, 3072, 3072, 1), (3001, 3072, 3072, 1), (40, 3072, 192, 1), (300, 3072, 200, 1), (512, 3072, 3072, 2)]
+          (1921, 3072, 3072, 1), (3001, 3072, 3072, 1), (64, 3072, 14336, 1), (50, 3072, 8968, 1), (129, 3072, 3072, 1),
+          (40, 3072, 192, 1), (300, 3072, 200, 1), (512, 3072, 3072, 2)]
 
 
 @pytest.mark.parametrize("M,K,N,nseg", SHAPES)

@@ -19,6 +19,7 @@ namespace wam {
 // helps; k ranges trade the second against partial-sum traffic.
 using Small32 = GemmCfg<32, 128, 64, 1, 4, 3, 2>;
 using Small64 = GemmCfg<64, 128, 64, 1, 4, 5>;
+using Small64n64 = GemmCfg<64, 64, 64, 2, 2, 5>;
 using Small128 = GemmCfg<128, 128, 64, 2, 4, 5, 1, 2>;
 using Small192 = GemmCfg<192, 128, 64, 2, 4, 3, 1, 2>;
 using Small256 = GemmCfg<256, 128, 64, 4, 2, 3, 1, 2>;
@@ -39,6 +40,9 @@ using Small256f8 = GemmCfg<256, 128, 64, 4, 2, 3, 1, 0, 1>;
 //   224 x 3072 x 3072  30 -> 18        1024 x 9216 x 3072 104 -> 60
 //   224 x 3072 x 14336 125 -> 37       1560 x 3072 x 14336 227 -> 122
 //   1024 x 1536 x 8960  82 -> 40       2325 x 3072 x 14336 218 -> 182
+// 64x64 tiles, against the best of the wider ones with their reduce pass (us):
+// 64 x 14336 x 3072 24.3 -> 21.7 and 32 rows 21.9 -> 18.8 (whole k on 224
+// CUs), 224 x 3072 x 3072 17.7 -> 14.8, 32 x 3072 x 3072 10.6 -> 9.6.
 // The four-wave kernel's tiles of 128 to 192 rows, against the best of the
 // others (us): 2325 x 3072 x 3072 51 -> 45, 1024 x 8960 x 1536 35 -> 31, 1024 x
 // 1536 x 8960 40.3 -> 39.5.  A reduction that a
@@ -51,8 +55,9 @@ struct TileCost {
 constexpr TileCost kTiles[] = {
     {32, 128, 0.3, 0.47},  {64, 128, 1.9, 0.42},  {128, 128, 3.0, 0.49}, {192, 128, 2.2, 0.64}, {256, 128, 2.7, 0.88},
     {128, 256, 2.3, 0.83}, {160, 256, 4.5, 0.90}, {192, 256, 6.0, 1.03}, {224, 256, 4.7, 1.05}, {256, 256, 4.4, 1.21},
+    {64, 64, 0.5, 0.28},
 };
-constexpr int kTile32 = 0, kTile192 = 3, kTileW4 = 5, kTileW224 = 8, kTileCount = 10;
+constexpr int kTile32 = 0, kTile192 = 3, kTileW4 = 5, kTileW224 = 8, kTile64n64 = 10, kTileCount = 11;
 constexpr double kHbmBytesPerUs = 6.6e6;
 constexpr int kMaxRanges = 32;
 
@@ -63,13 +68,13 @@ SplitPlan split_plan(int M, int seg_n, int n_seg, int K, int wb, int64_t ws_byte
   double best_cost = 1e30;
   for (int c = 0; c < kTileCount; ++c) {
     const TileCost& t = kTiles[c];
-    const bool w4 = c >= kTileW4;
+    const bool w4 = c >= kTileW4 && c < kTile64n64;
     // 256-column tiles hold whole tiles of one segment; the fp8-weight small
     // tiles are 128 columns wide
     if ((w4 && seg_n % 256 != 0) || (n_seg > 1 && seg_n % t.bn != 0)) continue;
     // fp8 weights: 64 and 128 rows, 256 x 128 (a 32-row stage would not hold a
     // 32-row slab of the fp32 epilogue), and the two largest
-    if (wb == 1 && (c == kTile32 || c == kTile192 || (w4 && c < kTileW224))) continue;
+    if (wb == 1 && (c == kTile32 || c == kTile192 || c == kTile64n64 || (w4 && c < kTileW224))) continue;
     // a shorter tile holds all rows
     if (c > (wb == 1 ? 1 : 0) && kTiles[c - 1].bm >= M && kTiles[c - 1].bn == t.bn) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((seg_n + t.bn - 1) / t.bn) * n_seg;
@@ -130,6 +135,7 @@ static int launch_small(LinearParams& p, hipStream_t s) {
 int split_tiles(LinearParams& p, const SplitPlan& g, int wb, hipStream_t s) {
   p.k_split = g.ks;
   WAM_REQUIRE(g.ks == 1 || (p.part && g.ks <= p.K / 64), "wam_linear: bad split-K launch");
+  if (g.tile == kTile64n64) return launch_small<Small64n64>(p, s);
   if (g.tile >= kTileW4) return w4_tiles(p, kTiles[g.tile].bm, wb, s);
   if (wb == 1) {
     switch (g.tile) {

@@ -351,7 +351,7 @@ __global__ __launch_bounds__(C::kThreads, C::BLOCKS) void gemm_bf16_kernel(Linea
   constexpr int NROUNDS = (C::BM + ROUND - 1) / ROUND;
   constexpr int QPR = C::BN / 4;                         // 16-byte chunks per fp32 row
   constexpr int RPI = 64 / QPR;                          // rows per wave-wide access
-  static_assert(QPR == 64 || QPR == 32, "BN must be 256 or 128");
+  static_assert(QPR == 64 || QPR == 32 || QPR == 16, "BN must be 256, 128 or 64");
   constexpr int ROW_B = C::BN * 4;
   void* out = seg == 0 ? p.out[0] : (seg == 1 ? p.out[1] : p.out[2]);
   const bf16* __restrict__ bias = seg == 0 ? p.bias[0] : (seg == 1 ? p.bias[1] : p.bias[2]);
