@@ -1128,7 +1128,9 @@ int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys) {
     const FewPlan p = attention_few_plan(b, m, H, max_keys, sharing, INT64_MAX);
     if (p.qw) most = std::max(most, attention_few_bytes(p, b, m, H));
   };
-  for (int sharing = 1; sharing <= 8; ++sharing) few(B, Mq, sharing);
+  few(B, Mq, 1);
+  for (int g = 2; g <= kFewGroupMax && g * (int64_t)Mq <= 32; ++g)
+    if (B % g == 0) few(B, Mq, g);
   if (B > 1 && (int64_t)B * Mq < (1 << 26)) few(1, B * Mq, 1);
   return most;
 }

@@ -35,6 +35,7 @@ __device__ inline float q_rms_factor(const wam_attention_args& a, int b, int qi)
   return rsqrtf(s / (float)a.q_norm_dim + a.q_eps);
 }
 
+constexpr int kFewGroupMax = 8;  // batch rows per group of attention_few_kernel
 // The kernel for calls with few queries per key source: query waves per
 // workgroup (1, 2 or 4 of 32 queries; 0: not this kernel), batch rows per
 // group and key-tile ranges (each a workgroup of its own, merged by a second

@@ -19,7 +19,6 @@ namespace wam {
 constexpr int kFewKeys = 32;                      // keys per tile
 constexpr int kFewTile = kFewKeys * kAttnHD * 2;  // 8 KB of K or V
 constexpr int kFewWaves = 8;
-constexpr int kFewGroupMax = 8;                   // batch rows per group
 constexpr int kFewMaxRanges = 8;
 
 // Maximum of three (a NaN in any gives NaN, as a score that is NaN must).

@@ -81,7 +81,7 @@ struct Layout {
   size_t h, h8, h8s, qkv, attn, x1, x2, ck, cv, act, slots, newslots, info, ssq, zeros, split, split_bytes, total;
 };
 
-static Layout layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
+static Layout make_layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
   Layout L{};
   const size_t R = (size_t)B * M;
   size_t off = 0;
@@ -124,6 +124,22 @@ static Layout layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
   L.split = take(L.split_bytes);
   L.total = off;
   return L;
+}
+
+// The last shape's layout is kept per thread: its plans take 5 us of host time,
+// and every layer of a model asks twice (the size, then the call).
+static Layout layout(int B, int M, int D, int F, int Bc, int Lc, int pool) {
+  struct Key {
+    int v[8];
+  };
+  const Key key{{B, M, D, F, Bc, Lc, pool, device_cu_count()}};
+  thread_local Key last{};
+  thread_local Layout kept;
+  if (memcmp(&key, &last, sizeof(key)) != 0) {
+    kept = make_layout(B, M, D, F, Bc, Lc, pool);
+    last = key;
+  }
+  return kept;
 }
 
 __global__ void cast_f32_bf16_kernel(const float* x, bf16* y, int64_t n) {
