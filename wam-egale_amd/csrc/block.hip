@@ -42,6 +42,7 @@ bool linear_norm_in_epilogue(int M, int seg_n, int n_seg, int K, int64_t ws_byte
 int kv_layout(const wam_kv_layout_args*, hipStream_t);
 int kv_layout_check(const wam_kv_layout_args*);
 int kv_commit(const wam_kv_commit_args*, hipStream_t);
+int kv_commit_check(const wam_kv_commit_args*);
 
 static thread_local char g_error[1024] = "";
 
@@ -435,16 +436,6 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     WAM_TRY(attention(&t, s));
   }
   WAM_TRY(copy_debug(a->debug, 4, attn, rowb, s));
-  // 6. New K/V into the pool for committed updates.
-  if (cache && !candidate && a->update != 0) {
-    Scope sc(a->timer, WAM_STAGE_KV_COMMIT, s);
-    wam_kv_commit_args c{};
-    c.k = qkv + D; c.v = qkv + 2 * D; c.ld = 3 * D;
-    c.pool_k = a->cache_k; c.pool_v = a->cache_v;
-    c.pool_bstride = (int64_t)a->pool * D; c.pool_rstride = D;
-    c.new_slots = newslots; c.B = B; c.tokens = M; c.D = D;
-    WAM_TRY(kv_commit(&c, s));
-  }
   // 7. Output projection + gated residual (gate 2).
   {
     Scope sc(a->timer, WAM_STAGE_SELF_OUT, s);
@@ -457,6 +448,18 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     if (W->w[1]) WAM_TRY(linear_partials(&g, s, &sp, &split));
     if (!split) WAM_TRY(linear(&g, s));
   }
+  // 6. New K/V into the pool for committed updates: by workgroups of the row
+  //    pass that reduces a split projection, or a launch.
+  wam_kv_commit_args c{};
+  const bool commit = cache && !candidate && a->update != 0;
+  if (commit) {
+    Scope sc(a->timer, WAM_STAGE_KV_COMMIT, s);
+    c.k = qkv + D; c.v = qkv + 2 * D; c.ld = 3 * D;
+    c.pool_k = a->cache_k; c.pool_v = a->cache_v;
+    c.pool_bstride = (int64_t)a->pool * D; c.pool_rstride = D;
+    c.new_slots = newslots; c.B = B; c.tokens = M; c.D = D;
+    WAM_TRY(split ? kv_commit_check(&c) : kv_commit(&c, s));
+  }
   // 8. norm2 (affine LayerNorm), or without cross_attn_norm the bf16 cast
   //    of the residual stream that the identity norm2 passes through.
   const bf16* n2 = h;
@@ -466,7 +469,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       wam_ln_args l{};
       l.x = x1; l.x_dtype = WAM_F32; l.y = h; l.rows = R; l.D = D; l.eps = W->eps[1]; l.affine = 1;
       l.gamma = W->w[1]; l.beta = W->w[2]; l.gb_dtype = W->norm2_dtype;
-      WAM_TRY(split ? split_ln(sp, l, s) : ln_modulate(&l, s));
+      WAM_TRY(split ? split_ln(sp, l, commit ? &c : nullptr, s) : ln_modulate(&l, s));
     } else {
       WAM_TRY(cast_f32_bf16(x1, h, (int64_t)R * D, s));
     }
@@ -561,7 +564,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
       l.y8 = h8; l.y8_scale = h8s;
       if (!dbg(12)) l.y = nullptr;
     }
-    WAM_TRY(split ? split_ln(sp, l, s) : ln_modulate(&l, s));
+    WAM_TRY(split ? split_ln(sp, l, nullptr, s) : ln_modulate(&l, s));
   }
   WAM_TRY(copy_debug(a->debug, 11, x2, rowb * 2, s));
   if (dbg(22)) WAM_TRY(plain_linear(attn, D, D, 19, -1, dbg(22)));

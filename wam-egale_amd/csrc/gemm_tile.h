@@ -58,7 +58,9 @@ int split_reduce(const LinearParams& p, int wb, hipStream_t s);
 // split_rms_rope or split_ln on *p).  Otherwise nothing is launched.
 int linear_partials(const wam_linear_args* a, hipStream_t s, LinearParams* p, bool* split);
 int split_rms_rope(const LinearParams& p, const wam_rms_rope_args& r, const wam_kv_layout_args* kv, hipStream_t s);
-int split_ln(const LinearParams& p, const wam_ln_args& l, hipStream_t s);
+// commit (may be null): the new K/V rows' copy to the pool, by workgroups of
+// the same launch (the gated residual without fp8 rows).
+int split_ln(const LinearParams& p, const wam_ln_args& l, const wam_kv_commit_args* commit, hipStream_t s);
 // One launch of the four-wave kernel on tm-row tiles (128 to 256; fp8 weights
 // 224 or 256); with p.k_split > 1 its partial sums only.
 int w4_tiles(LinearParams& p, int tm, int wb, hipStream_t s);

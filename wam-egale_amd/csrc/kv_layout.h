@@ -174,4 +174,23 @@ __device__ inline void kv_layout_pool(const wam_kv_layout_args& a) {
   }
 }
 
+// New K/V rows to their pool slots, 16 bytes a thread and step, by `blocks`
+// workgroups of T threads.
+template <int T>
+__device__ inline void kv_commit_rows(const wam_kv_commit_args& a, int block, int blocks) {
+  const int chunks = a.D >> 3;
+  const int64_t n = (int64_t)a.B * a.tokens * chunks;
+  for (int64_t i = (int64_t)block * T + threadIdx.x; i < n; i += (int64_t)blocks * T) {
+    int64_t row, cc;
+    split_row(i, chunks, row, cc);  // i < 2^31: B * tokens * D / 8 elements
+    const int c = (int)cc;
+    int64_t b, t;
+    split_row(row, a.tokens, b, t);
+    const int64_t src = row * a.ld + c * 8;
+    const int64_t dst = b * a.pool_bstride + (int64_t)a.new_slots[t] * a.pool_rstride + c * 8;
+    st_bf16x8(static_cast<bf16*>(a.pool_k) + dst, ld_bf16x8(static_cast<const bf16*>(a.k) + src));
+    st_bf16x8(static_cast<bf16*>(a.pool_v) + dst, ld_bf16x8(static_cast<const bf16*>(a.v) + src));
+  }
+}
+
 }  // namespace wam
