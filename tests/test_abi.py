@@ -245,3 +245,13 @@ def test_small_grid_plan_workspace():
     assert h.wam_linear_workspace_bytes(32, 3072, 1, 14336) == 5 * 32 * 3072 * 4
     assert h.wam_linear_workspace_bytes(224, 3072, 1, 14336) == 5 * 224 * 3072 * 4
     assert h.wam_linear_workspace_bytes(224, 14336, 1, 3072) == 0
+
+
+def test_block_workspace_of_empty_shapes():
+    """A size is answered for every shape, empty ones too (the block itself
+    refuses them, with a message); each shape in turn, so that no layout kept
+    from the one before answers for it."""
+    h = _lib.lib()
+    for shape in ((1, 0, 256, 512, 1, 20, 0), (0, 60, 256, 512, 1, 20, 0), (1, 60, 256, 0, 1, 20, 0),
+                  (1, 60, 256, 512, 0, 0, 0), (1, 60, 256, 512, 1, 0, 0), (0, 0, 0, 0, 0, 0, 0)):
+        assert 0 <= h.wam_block_workspace_bytes(*shape) < 1 << 24, shape

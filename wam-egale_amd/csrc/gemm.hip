@@ -1030,12 +1030,13 @@ int64_t linear_workspace_bytes(int M, int seg_n, int n_seg, int K) {
 
 // What linear_partials can use.
 int64_t linear_partials_bytes(int M, int seg_n, int n_seg, int K) {
-  if (K % 64 != 0 || uses_big_tiles(M, seg_n, n_seg)) return 0;
+  if (M < 1 || seg_n < 1 || K < 1 || K % 64 != 0 || uses_big_tiles(M, seg_n, n_seg)) return 0;
   return split_plan_bytes(split_plan(M, seg_n, n_seg, K, 2, INT64_MAX, true), M, seg_n, n_seg);
 }
 
 // What a launch with fp8 activations can use.
 int64_t linear_f8mm_bytes(int M, int N, int K) {
+  if (M < 1 || N < 1 || K < 1) return 0;
   return N % 256 == 0 && K % 128 == 0 ? split_plan_bytes(f8mm_plan(M, N, K, INT64_MAX), M, N, 1) : 0;
 }
 
