@@ -100,6 +100,19 @@ def test_attention_host_validation():
     assert "bad shape" in _err(h.wam_attention(ctypes.byref(a), None))
 
 
+def test_attention_contract_before_plan():
+    """Both entry points refuse a pool without batch rows before they plan
+    with their number."""
+    h = _lib.lib()
+    a = _lib.AttentionArgs()
+    a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch = 2, 4, 1, 128, 4, 2
+    a.q = a.o = a.k = a.v = a.pool_k = a.pool_v = a.slots = a.n_hist_dev = a.pool_rows = 16
+    a.q_rstride = a.o_rstride = a.kv_rstride = a.pool_rstride = a.pool_bstride = 128
+    a.q_bstride = a.o_bstride = a.kv_bstride = 512
+    for f in (h.wam_attention, h.wam_attention_noalloc):
+        assert "pool_batch" in _err(f(ctypes.byref(a), None))
+
+
 def test_kv_layout_host_validation():
     h = _lib.lib()
     a = _lib.KvLayoutArgs()

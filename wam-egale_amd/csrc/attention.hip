@@ -1135,7 +1135,9 @@ int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys) {
   return most;
 }
 
-int attention(const wam_attention_args* a, hipStream_t s) {
+// The contract of a call; whatever plans one (a division by a batch count,
+// say) comes after it.
+static int attention_check(const wam_attention_args* a) {
   WAM_REQUIRE(a != nullptr, "wam_attention: null args");
   WAM_REQUIRE(a->head_dim == kAttnHD, "wam_attention: head_dim must be 128 (got %d)", a->head_dim);
   WAM_REQUIRE(a->B >= 1 && a->H >= 1 && a->Mq >= 0 && a->Mk >= 1,
@@ -1162,6 +1164,11 @@ int attention(const wam_attention_args* a, hipStream_t s) {
   WAM_REQUIRE(!a->q_ssq || (a->q_ssq_n >= 1 && a->q_ssq_n <= kQssqMax && a->q_norm_dim >= 1),
               "wam_attention: q_ssq needs 1..%d partials per row and q_norm_dim >= 1 (got %d, %d)", kQssqMax,
               a->q_ssq_n, a->q_norm_dim);
+  return WAM_OK;
+}
+
+int attention(const wam_attention_args* a, hipStream_t s) {
+  WAM_TRY(attention_check(a));
   if (a->Mq == 0) return WAM_OK;
   wam_attention_args call;
   FewPlan few;
@@ -1253,6 +1260,7 @@ int attention_noalloc(const wam_attention_args* a, hipStream_t s) {
               "wam_attention_noalloc: takes no workspace (the split uses the library's own scratch)");
   WAM_REQUIRE(a->B >= 1 && a->H >= 1 && a->Mq >= 0 && a->Mk >= 1 && a->max_keys >= 0,
               "wam_attention_noalloc: bad shape B=%d H=%d Mq=%d Mk=%d", a->B, a->H, a->Mq, a->Mk);
+  WAM_TRY(attention_check(a));
   // The split wam_attention would run with an unlimited workspace; shapes
   // whose partial results exceed the scratch are refused, not re-planned, so
   // that both entry points compute the same thing.
