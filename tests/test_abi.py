@@ -113,6 +113,18 @@ def test_attention_contract_before_plan():
         assert "pool_batch" in _err(f(ctypes.byref(a), None))
 
 
+# Shapes whose count of 32-, 64- or 128-query units passes 2^31 or 2^32.
+@pytest.mark.parametrize("B,Mq,H", [(1 << 20, 32768, 24), (1 << 20, 16384, 32), (1 << 18, 32767, 64)])
+def test_attention_refuses_huge_grids(B, Mq, H):
+    h = _lib.lib()
+    a = _lib.AttentionArgs()
+    a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch = B, Mq, H, 128, 512, 1
+    a.q = a.o = a.k = a.v = 16
+    a.q_rstride = a.o_rstride = a.kv_rstride = 128
+    assert "grid too large" in _err(h.wam_attention(ctypes.byref(a), None))
+    assert h.wam_attention_workspace_bytes(B, Mq, H, 512) == 0
+
+
 def test_kv_layout_host_validation():
     h = _lib.lib()
     a = _lib.KvLayoutArgs()

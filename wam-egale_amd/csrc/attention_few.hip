@@ -375,12 +375,14 @@ __global__ __launch_bounds__(256) void few_combine_kernel(wam_attention_args a, 
                              (int64_t)(vq - bl * a.Mq) * a.o_rstride + h * kAttnHD + 2 * lane) = r;
 }
 
-static int few_units(int qw, int group, int B, int Mq, int H) {
-  return (group * Mq + 32 * qw - 1) / (32 * qw) * (B / group) * H;
+// (64-bit: the size query and the plan take any shape, a launch has at most a
+// dispatch round of units)
+static int64_t few_units(int qw, int group, int B, int Mq, int H) {
+  return ((int64_t)group * Mq + 32 * qw - 1) / (32 * qw) * (B / group) * H;
 }
 
 int64_t attention_few_bytes(const FewPlan& p, int B, int Mq, int H) {
-  return p.ranges > 1 ? (int64_t)p.ranges * few_units(p.qw, p.group, B, Mq, H) * 32 * p.qw * (kAttnHD + 2) * 4 : 0;
+  return p.ranges > 1 ? p.ranges * few_units(p.qw, p.group, B, Mq, H) * 32 * p.qw * (kAttnHD + 2) * 4 : 0;
 }
 
 // The workgroups must fit one dispatch round (one per CU): more queries per
@@ -406,7 +408,7 @@ FewPlan attention_few_plan(int B, int Mq, int H, int64_t keys, int sharing, int6
   const int tiles = (int)((keys + kFewKeys - 1) / kFewKeys);
   for (int qw = 1; qw <= 4; qw *= 2) {
     const int g = qw == 1 ? group : 1;
-    const int units = few_units(qw, g, B, Mq, H);
+    const int64_t units = few_units(qw, g, B, Mq, H);
     if (units > cus || (qw > 1 && Mq <= 16 * qw)) continue;
     for (int r = 1; r <= kFewMaxRanges && units * r <= cus; ++r) {
       if (r > 1 && r * kFewWaves / qw > tiles) break;
@@ -423,7 +425,7 @@ FewPlan attention_few_plan(int B, int Mq, int H, int64_t keys, int sharing, int6
 }
 
 int attention_few(const wam_attention_args* a, const FewPlan& p, float* part, hipStream_t s) {
-  const int QB = 32 * p.qw, units = few_units(p.qw, p.group, a->B, a->Mq, a->H);
+  const int QB = 32 * p.qw, units = (int)few_units(p.qw, p.group, a->B, a->Mq, a->H);
   const dim3 grid((unsigned)(units * p.ranges)), block(64 * kFewWaves);
   auto kernel = p.qw == 4   ? attention_few_kernel<4, false>
                 : p.qw == 2 ? attention_few_kernel<2, false>
