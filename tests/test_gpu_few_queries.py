@@ -134,6 +134,41 @@ def test_workspace_sizes(dev, B, Mq, Mk):
     assert torch.equal(outs[2], outs[3])
 
 
+# Few keys, where the two kernels' predicted times are close: own keys only,
+# and most of them in a pool.
+@pytest.mark.parametrize("H", [12, 24])
+@pytest.mark.parametrize("Mq", [1, 17, 33, 49, 60, 120])
+def test_entry_points_agree(dev, Mq, H):
+    """wam_attention with its whole workspace and the entry point without
+    allocation run the same kernel: equal bits."""
+    from wam_ops import _lib
+    h = _lib.lib()
+    for keys in (32, 64, 128, 192, 300):
+        for n in (0, keys - min(Mq, keys - 1)):
+            own = keys - n
+            q, k, v = _randn((1, Mq, H, 128), dev, 1), _randn((1, own, H, 128), dev, 2), _randn((1, own, H, 128), dev, 3)
+            kw = _pool(dev, 1, max(n, 1), H, torch.arange(n, device=dev), 4)
+            outs = []
+            for f in (h.wam_attention, h.wam_attention_noalloc):
+                o = torch.zeros_like(q)
+                a = _lib.AttentionArgs()
+                a.q, a.q_bstride, a.q_rstride = q.data_ptr(), q.stride(0), q.stride(1)
+                a.o, a.o_bstride, a.o_rstride = o.data_ptr(), o.stride(0), o.stride(1)
+                a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch, a.scale, a.max_keys = 1, Mq, H, 128, own, 1, 128 ** -0.5, keys
+                a.k, a.v, a.kv_bstride, a.kv_rstride = k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1)
+                if n:
+                    a.pool_k, a.pool_v, a.pool_batch = kw["pool_k"].data_ptr(), kw["pool_v"].data_ptr(), 1
+                    a.pool_bstride, a.pool_rstride = n * H * 128, H * 128
+                    a.slots, a.n_hist_dev, a.hist_base_dev = (kw[x].data_ptr() for x in ("slots", "n_hist", "hist_base"))
+                if not outs:
+                    ws = torch.empty(h.wam_attention_workspace_bytes(1, Mq, H, keys) + 16, dtype=torch.uint8, device=dev)
+                    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+                _lib.check(f(ctypes.byref(a), None), "wam_attention")
+                torch.cuda.synchronize()
+                outs.append(o)
+            assert torch.equal(*outs), (Mq, H, keys, n)
+
+
 def test_candidates_are_isolated(dev):
     """A candidate whose own rows hold infinities and NaN leaves the others,
     its neighbour in the same workgroup too, as they were."""

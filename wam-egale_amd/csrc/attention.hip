@@ -1167,13 +1167,8 @@ static int attention_check(const wam_attention_args* a) {
   return WAM_OK;
 }
 
-int attention(const wam_attention_args* a, hipStream_t s) {
-  WAM_TRY(attention_check(a));
-  if (a->Mq == 0) return WAM_OK;
-  wam_attention_args call;
-  FewPlan few;
-  if (takes_few(a, a->workspace ? a->workspace_bytes : 0, &call, &few))
-    return attention_few(&call, few, static_cast<float*>(a->workspace), s);
+// A call that the few-query kernel does not take.
+static int attention_units(const wam_attention_args* a, hipStream_t s) {
   // 8 or 7 waves (256 or 224 queries) per workgroup, with the last dispatch
   // round split by key ranges when the plan says so and the caller gave a
   // workspace for the partial results; small grids use 4-wave workgroups.
@@ -1222,6 +1217,16 @@ int attention(const wam_attention_args* a, hipStream_t s) {
   return WAM_OK;
 }
 
+int attention(const wam_attention_args* a, hipStream_t s) {
+  WAM_TRY(attention_check(a));
+  if (a->Mq == 0) return WAM_OK;
+  wam_attention_args call;
+  FewPlan few;
+  if (takes_few(a, a->workspace ? a->workspace_bytes : 0, &call, &few))
+    return attention_few(&call, few, static_cast<float*>(a->workspace), s);
+  return attention_units(a, s);
+}
+
 // ------------------------------------------------------------ no allocation
 // wam_attention for callers that cannot allocate device memory (code under
 // HIP graph capture, tight serving loops): the key-range split's partial
@@ -1261,30 +1266,32 @@ int attention_noalloc(const wam_attention_args* a, hipStream_t s) {
   WAM_REQUIRE(a->B >= 1 && a->H >= 1 && a->Mq >= 0 && a->Mk >= 1 && a->max_keys >= 0,
               "wam_attention_noalloc: bad shape B=%d H=%d Mq=%d Mk=%d", a->B, a->H, a->Mq, a->Mk);
   WAM_TRY(attention_check(a));
-  // The split wam_attention would run with an unlimited workspace; shapes
-  // whose partial results exceed the scratch are refused, not re-planned, so
-  // that both entry points compute the same thing.
+  if (a->Mq == 0) return WAM_OK;
+  // The kernel and the split that wam_attention runs with an unlimited
+  // workspace (as much as wam_attention_workspace_bytes asks for never limits
+  // it), chosen once, so that both entry points compute the same thing.
+  // Shapes whose partial results exceed the scratch are refused, not
+  // re-planned.
   const int64_t keys = a->max_keys > 0 ? a->max_keys : a->Mk;
-  int64_t need =
-      a->Mq > 0 ? plan_bytes(attention_plan(a->B, a->Mq, a->H, keys, INT64_MAX, query_tile(a, keys))) : 0;
+  int64_t need = plan_bytes(attention_plan(a->B, a->Mq, a->H, keys, INT64_MAX, query_tile(a, keys)));
   WAM_REQUIRE(need <= kNoAllocScratchBytes,
               "wam_attention_noalloc: this shape's key-range split needs %lld bytes of scratch, more than "
               "the %lld-byte maximum; call wam_attention with a workspace instead",
               (long long)need, (long long)kNoAllocScratchBytes);
-  // (the few-query kernel's ranges, at most 256 partial tiles of 128 queries,
-  // always fit)
   wam_attention_args call;
   FewPlan few;
-  if (a->Mq > 0 && takes_few(a, kNoAllocScratchBytes, &call, &few))
-    need = attention_few_bytes(few, call.B, call.Mq, call.H);
-  wam_attention_args b = *a;
-  if (need > 0) {
-    void* p = nullptr;
-    WAM_TRY(scratch_address(&p));
-    b.workspace = p;
-    b.workspace_bytes = need;
-  }
-  return attention(&b, s);
+  const bool few_queries = takes_few(a, INT64_MAX, &call, &few);
+  // (the few-query kernel's ranges, at most one partial tile of 128 queries
+  // per CU, fit in 17 MB of 256 CUs)
+  if (few_queries) need = attention_few_bytes(few, call.B, call.Mq, call.H);
+  WAM_REQUIRE(need <= kNoAllocScratchBytes, "wam_attention_noalloc: %lld bytes of scratch", (long long)need);
+  void* p = nullptr;
+  if (need > 0) WAM_TRY(scratch_address(&p));
+  if (few_queries) return attention_few(&call, few, static_cast<float*>(p), s);
+  call = *a;
+  call.workspace = p;
+  call.workspace_bytes = need;
+  return attention_units(&call, s);
 }
 
 }  // namespace wam
