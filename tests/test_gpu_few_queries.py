@@ -90,6 +90,26 @@ def test_pool(dev, B, Mq, n, gap, rows):
     assert_close(ops.attention(q, k, v, **kw), _ref(q, k, v, src), 2e-2, 0.9999, f"pool {B}x{Mq} over {n}")
 
 
+@pytest.mark.parametrize("gap", [0, 9])
+def test_pool_of_one_row(dev, gap):
+    """A pool [1, P, H, hd] is contiguous whatever the stride of its first
+    dimension: a transposed [P, 1, H, hd] has that of one slot."""
+    from wam_ops import ops
+    Mq, n, H = 16, 300, 24
+    q, k, v = _randn((1, Mq, H, 128), dev, 1, 2.0), _randn((1, Mq, H, 128), dev, 2), _randn((1, Mq, H, 128), dev, 3)
+    valid = torch.arange(n, device=dev)
+    valid[n // 2:] += gap
+    kw = _pool(dev, 1, n + 20, H, valid, 4)
+    ref = _ref(q, k, v, [(torch.cat([kw["pool_k"][0, valid], k[0]]), torch.cat([kw["pool_v"][0, valid], v[0]]))])
+    for x in ("pool_k", "pool_v"):
+        rows = kw[x].new_empty(n + 20, 1, H, 128)
+        rows[:, 0] = kw[x][0]
+        kw[x] = rows.transpose(0, 1)
+        assert kw[x].is_contiguous()
+        assert kw[x].stride(0) == H * 128
+    assert_close(ops.attention(q, k, v, **kw), ref, 2e-2, 0.9999, f"pool of one row, gap {gap}")
+
+
 def test_own_row_map_and_query_rms(dev):
     """kv_rows, and q_ssq's per-query factor (rows of the folded batch too)."""
     from wam_ops import ops

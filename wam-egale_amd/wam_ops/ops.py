@@ -355,7 +355,9 @@ def attention(q, k, v, *, pool_k=None, pool_v=None, slots=None, n_hist=None, poo
             _bf16(t, "pool")
             _req(t.is_contiguous() and t.shape[2:] == (H, hd), "pool must be [Bp, P, H, 128]")
         a.pool_k, a.pool_v = pool_k.data_ptr(), pool_v.data_ptr()
-        a.pool_bstride, a.pool_rstride = pool_k.stride(0), pool_k.stride(1)
+        # (a contiguous pool of one row may carry any stride for that dimension)
+        a.pool_rstride = H * hd
+        a.pool_bstride = pool_k.shape[1] * a.pool_rstride
         a.pool_batch = pool_k.shape[0]
         a.slots, a.n_hist_dev = slots.data_ptr(), n_hist.data_ptr()
         if hist_base is not None:
