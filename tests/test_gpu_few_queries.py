@@ -110,6 +110,28 @@ def test_pool_of_one_row(dev, gap):
     assert_close(ops.attention(q, k, v, **kw), ref, 2e-2, 0.9999, f"pool of one row, gap {gap}")
 
 
+# One, two and four query waves, and groups: the first keys some wave sees.
+@pytest.mark.parametrize("B,Mq,Mk,rows", [(1, 16, 300, None), (1, 50, 300, None), (1, 200, 300, None),
+                                          (14, 16, 100, [0] * 14)])
+def test_scores_of_minus_infinity(dev, B, Mq, Mk, rows):
+    """Keys whose scores are -inf have no weight, whole tiles of them too."""
+    from wam_ops import ops
+    H, dead = 24, slice(32, 96)
+    q = _randn((B, Mq, H, 128), dev, 1).abs() + 0.1
+    k, v = _randn((B, Mk, H, 128), dev, 2), _randn((B, Mk, H, 128), dev, 3)
+    keep = torch.ones(Mk, dtype=torch.bool, device=dev)
+    keep[dead] = False
+    src = [(k[b, keep], v[b, keep]) for b in range(B)]
+    kw = {}
+    if rows:
+        kw = _pool(dev, 1, 70, H, torch.arange(70, device=dev), 4)
+        kw["pool_rows"] = torch.tensor(rows, device=dev)
+        src = [(torch.cat([kw["pool_k"][0], a]), torch.cat([kw["pool_v"][0], b])) for a, b in src]
+    ref = _ref(q, k, v, src)
+    k[:, dead] = float("-inf")
+    assert_close(ops.attention(q, k, v, **kw), ref, 2e-2, 0.9999, f"scores of -inf {B}x{Mq}x{Mk}")
+
+
 def test_own_row_map_and_query_rms(dev):
     """kv_rows, and q_ssq's per-query factor (rows of the folded batch too)."""
     from wam_ops import ops

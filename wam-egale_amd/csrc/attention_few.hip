@@ -21,6 +21,10 @@ constexpr int kFewTile = kFewKeys * kAttnHD * 2;  // 8 KB of K or V
 constexpr int kFewWaves = 8;
 constexpr int kFewMaxRanges = 8;
 
+// Running maximum of a query without a finite score: finite, so that a score
+// of -inf less it is -inf (less -inf it would be NaN), and below any other.
+constexpr float kNoMax = -__FLT_MAX__;
+
 // Maximum of three (a NaN in any gives NaN, as a score that is NaN must).
 __device__ inline float max3(float a, float b, float c) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attention_few_kernel(wam_at
   const int tr_i = lane & 15, tr_gh = (lane >> 4) & 1;
   const int kfrag0 = k_off(l32, half), vfrag0 = v_off(4 * half + (tr_i >> 2), 2 * tr_gh + ((tr_i & 3) >> 1)) + (tr_i & 1) * 8;
   const int krow0 = lrow * 256 + ((pch ^ (lane >> 4)) << 4), vrow = v_off(lrow, pch);
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = kNoMax, l_run = 0.f;
   f32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
@@ -212,7 +216,8 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attention_few_kernel(wam_at
     }
     // Lazy rescaling as in attention_kernel: the running max (log2 units,
     // equal in both lane halves of a query) moves by more than 8 or not at
-    // all.  It stays -inf while the query has seen no key of its own.
+    // all.  It stays at kNoMax while the query has seen scores of -inf only
+    // (another row's keys among them), whose weights are then zeros.
     float mx = max3(max3(max3(s[0], s[1], s[2]), max3(s[3], s[4], s[5]), max3(s[6], s[7], s[8])),
                     max3(s[9], s[10], s[11]), max3(max3(s[12], s[13], s[14]), s[15], s[15]));
     if (__builtin_amdgcn_ballot_w64(mx * sc > m_run + 8.0f)) {
@@ -225,11 +230,10 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attention_few_kernel(wam_at
       for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
       m_run = m_new;
     }
-    const float m_sub = GROUP && !mine ? 0.f : m_run;
     bf16x8 pb[2];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      pb[v >> 3][v & 7] = static_cast<bf16>(__builtin_amdgcn_exp2f(s[v] * sc - m_sub));
+      pb[v >> 3][v & 7] = static_cast<bf16>(__builtin_amdgcn_exp2f(s[v] * sc - m_run));
     }
     // the sum of the weights O accumulates
     const bf16x2 one = {static_cast<bf16>(1.f), static_cast<bf16>(1.f)};
@@ -283,22 +287,19 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attention_few_kernel(wam_at
   // Merge over the KW key waves of a query block: each wave scales its O by
   // 2^(m - max m), the rows [query][d] go through LDS (16-byte chunks
   // XOR-swizzled by the query) and are summed.  A wave without a tile has m =
-  // -inf, l = 0, O = 0.
+  // kNoMax, l = 0, O = 0.
   const float l = l_run + __shfl_xor(l_run, 32, 64);
   if (half == 0) {
     s_ml[0][wave][l32] = m_run;
     s_ml[1][wave][l32] = l;
   }
   __syncthreads();
-  float m = -INFINITY, den = 0.f;
+  float m = kNoMax, den = 0.f;
 #pragma unroll
   for (int w = 0; w < KW; ++w) m = fmaxf(m, s_ml[0][w * QW + qw][l32]);
 #pragma unroll
-  for (int w = 0; w < KW; ++w) {
-    const float mw = s_ml[0][w * QW + qw][l32];
-    den += mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - m) * s_ml[1][w * QW + qw][l32];
-  }
-  const float scale = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m);
+  for (int w = 0; w < KW; ++w) den += __builtin_amdgcn_exp2f(s_ml[0][w * QW + qw][l32] - m) * s_ml[1][w * QW + qw][l32];
+  const float scale = __builtin_amdgcn_exp2f(m_run - m);
   const float f = ranges > 1 ? scale : scale / den;
   char* const ob = lds + wave * 2 * kFewTile;
 #pragma unroll
