@@ -132,6 +132,23 @@ def test_scores_of_minus_infinity(dev, B, Mq, Mk, rows):
     assert_close(ops.attention(q, k, v, **kw), ref, 2e-2, 0.9999, f"scores of -inf {B}x{Mq}x{Mk}")
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.05])
+@pytest.mark.parametrize("B,n,own", [(14, 304, 16), (1, 0, 128)])
+def test_scales_not_above_zero(dev, scale, B, n, own):
+    """Any scale, over whole 64-key tiles; candidates whose masks count."""
+    from wam_ops import ops
+    Mq, H = 16, 24
+    q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, own, H, 128), dev, 2), _randn((B, own, H, 128), dev, 3)
+    src, kw = list(zip(k, v)), {}
+    if n:
+        rows = [b // 7 for b in range(B)]
+        kw = _pool(dev, 2, n, H, torch.arange(n, device=dev), 4)
+        src = [(torch.cat([kw["pool_k"][r], a]), torch.cat([kw["pool_v"][r], b])) for r, (a, b) in zip(rows, src)]
+        kw["pool_rows"] = torch.tensor(rows, device=dev)
+    ref = _ref(q.float() * (scale * 128 ** 0.5), k, v, src)
+    assert_close(ops.attention(q, k, v, scale=scale, **kw), ref, 2e-2, 0.9999, f"scale {scale}, {B}x{Mq}")
+
+
 def test_own_row_map_and_query_rms(dev):
     """kv_rows, and q_ssq's per-query factor (rows of the folded batch too)."""
     from wam_ops import ops

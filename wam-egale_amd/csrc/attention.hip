@@ -1105,6 +1105,7 @@ static double plan_us(const wam_attention_args* a, int64_t keys, int64_t ws_byte
 // run of B * Mq queries (14 x 16 queries over one text context: whole waves).
 static bool takes_few(const wam_attention_args* a, int64_t ws_bytes, wam_attention_args* call, FewPlan* few) {
   const int64_t keys = a->max_keys > 0 ? a->max_keys : a->Mk;
+  if (!(a->scale > 0.f)) return false;  // masked scores are -inf before the scale
   if (((int64_t)a->Mk + 64) * a->kv_rstride * 2 >= (int64_t)INT32_MAX) return false;
   if (a->n_hist_dev && (a->pool_bstride < a->pool_rstride || a->pool_bstride * 2 >= (int64_t)INT32_MAX)) return false;
   *call = *a;
