@@ -228,6 +228,23 @@ def test_entry_points_agree(dev, Mq, H):
             assert torch.equal(*outs), (Mq, H, keys, n)
 
 
+@pytest.mark.parametrize("B", [1, 6])  # fewer units than the pipelined kernel takes, and enough
+def test_backward_keys(dev, B):
+    """Own keys addressed from their last row back (a negative row stride)."""
+    from wam_ops import _lib
+    H, Mq, Mk = 24, 16, 200
+    q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, Mk, H, 128), dev, 2), _randn((B, Mk, H, 128), dev, 3)
+    ref, o = _ref(q, k, v, list(zip(k, v))), torch.zeros_like(q)
+    a = _lib.AttentionArgs()
+    a.q, a.q_bstride, a.q_rstride = q.data_ptr(), q.stride(0), q.stride(1)
+    a.o, a.o_bstride, a.o_rstride = o.data_ptr(), o.stride(0), o.stride(1)
+    a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch, a.scale = B, Mq, H, 128, Mk, B, 128 ** -0.5
+    a.k, a.v, a.kv_bstride, a.kv_rstride = k[0, -1].data_ptr(), v[0, -1].data_ptr(), k.stride(0), -k.stride(1)
+    _lib.check(_lib.lib().wam_attention(ctypes.byref(a), None), "wam_attention")
+    torch.cuda.synchronize()
+    assert_close(o, ref, 2e-2, 0.9999, f"backward keys {B}x{Mq}x{Mk}")
+
+
 def test_candidates_are_isolated(dev):
     """A candidate whose own rows hold infinities and NaN leaves the others,
     its neighbour in the same workgroup too, as they were."""

@@ -1053,15 +1053,21 @@ static AttnPlan attention_plan(int B, int Mq, int H, int64_t keys, int64_t max_b
 // measurement; always on in the library).
 static bool g_attn_w4 = true;
 
+// Whether `rows` rows from the first on lie within a 31-bit byte offset (rows
+// that go backwards, a negative stride, do not: they need 64-bit addresses).
+static bool rows_in_31_bits(int64_t rows, int64_t rstride) {
+  return rstride >= 0 && rows * rstride * 2 < (int64_t)INT32_MAX;
+}
+
 // The pipelined kernel runs when every Q and own K/V row's byte offset fits in
 // 31 bits, the pool rows of one batch row (slots < pool_bstride /
 // pool_rstride) in 32 bits, and the query grid is at least 128 units of 256
 // rows; smaller grids use attention_kernel<4>.
 static bool sp_eligible(const wam_attention_args* a) {
   const int64_t grid8 = (int64_t)((a->Mq + 255) / 256) * a->H * a->B;
-  return g_attn_w4 && grid8 >= 128 && ((int64_t)a->Mq + 256) * a->q_rstride * 2 < (int64_t)INT32_MAX &&
-         ((int64_t)a->Mk + kAttnKT) * a->kv_rstride * 2 < (int64_t)INT32_MAX &&
-         (!a->n_hist_dev || (a->pool_bstride >= a->pool_rstride && a->pool_bstride * 2 < (int64_t)UINT32_MAX));
+  return g_attn_w4 && grid8 >= 128 && rows_in_31_bits((int64_t)a->Mq + 256, a->q_rstride) &&
+         rows_in_31_bits((int64_t)a->Mk + kAttnKT, a->kv_rstride) &&
+         (!a->n_hist_dev || (a->pool_rstride >= 0 && a->pool_bstride >= a->pool_rstride && a->pool_bstride * 2 < (int64_t)UINT32_MAX));
 }
 
 // Query rows per unit of the pipelined kernel: 224 (7 waves) when its plan
@@ -1106,8 +1112,10 @@ static double plan_us(const wam_attention_args* a, int64_t keys, int64_t ws_byte
 static bool takes_few(const wam_attention_args* a, int64_t ws_bytes, wam_attention_args* call, FewPlan* few) {
   const int64_t keys = a->max_keys > 0 ? a->max_keys : a->Mk;
   if (!(a->scale > 0.f)) return false;  // masked scores are -inf before the scale
-  if (((int64_t)a->Mk + 64) * a->kv_rstride * 2 >= (int64_t)INT32_MAX) return false;
-  if (a->n_hist_dev && (a->pool_bstride < a->pool_rstride || a->pool_bstride * 2 >= (int64_t)INT32_MAX)) return false;
+  if (!rows_in_31_bits((int64_t)a->Mk + 64, a->kv_rstride)) return false;
+  if (a->n_hist_dev && (a->pool_rstride < 0 || a->pool_bstride < a->pool_rstride ||
+                        a->pool_bstride * 2 >= (int64_t)INT32_MAX))
+    return false;
   *call = *a;
   if (a->B > 1 && !a->n_hist_dev && !a->kv_rows && a->kv_batch == 1 && a->q_bstride == a->Mq * a->q_rstride &&
       a->o_bstride == a->Mq * a->o_rstride && (int64_t)a->B * a->Mq < (1 << 26)) {
