@@ -91,3 +91,19 @@ def test_rope_table_batch_is_refused(dev, monkeypatch):
         with torch.no_grad(), pytest.raises(RuntimeError, match="freq batch"):
             blk(x, ctx, temb, freqs[:1].expand(3, *freqs.shape[1:]))
     torch.cuda.synchronize()
+
+
+def test_calls_go_to_the_current_stream(dev):
+    """The handle the operators launch on is the current stream's, and a
+    call's scratch outlives its work on a side stream."""
+    from wam_ops import ops
+    x, w = (_randn(s, dev, i, 0.1, torch.bfloat16) for i, s in enumerate(((32, 1536), (1536, 1536))))
+    ref = ops.linear(x, w)
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        assert ops.stream_handle(dev).value == side.cuda_stream
+        outs = [ops.linear(x, w) for _ in range(8)]
+    assert (ops.stream_handle(dev).value or 0) == torch.cuda.current_stream(dev).cuda_stream
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, ref) for o in outs)

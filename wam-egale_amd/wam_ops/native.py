@@ -228,8 +228,8 @@ def run_block(bound, hidden_states, encoder_hidden_states, temb, rotary_emb, cac
         args.timer = timer
     _lib.check(_lib.lib().wam_block_forward(ctypes.byref(args), stream_handle(dev)),
                "wam_block_forward")
-    # Keep the transient buffers alive until the stream has consumed them.
-    ws.record_stream(torch.cuda.current_stream(dev))
+    if ws is workspace:  # a caller's buffer: it may belong to another stream
+        ws.record_stream(torch.cuda.current_stream(dev))
     if debug:
         dbg["output"] = out
         return out, dbg

@@ -37,8 +37,15 @@ def dtype_code(t):
     raise RuntimeError(f"unsupported dtype {t.dtype} (need float32 or bfloat16)")
 
 
+# The current stream's handle without a Stream object (1.8 us of host time a
+# call, of 14 for a small linear).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is None or device.index is None:
+        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(_raw_stream(device.index))
 
 
 def _dev(*ts):
@@ -54,7 +61,8 @@ def _dev(*ts):
 
 
 def _bf16(t, name):
-    _req(t.dtype == torch.bfloat16, f"{name} must be bfloat16 (got {t.dtype})")
+    if t.dtype != torch.bfloat16:
+        raise RuntimeError(f"{name} must be bfloat16 (got {t.dtype})")
 
 
 def modulation(table, temb, tokens):
@@ -237,15 +245,13 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
         _req(table is not None and temb is not None and gate_index is not None, "gate needs table/temb")
         a.gate = modulation(table, temb, tokens if tokens is not None else M)
         a.gate_index = gate_index
-    scratch = None
     nbytes = _lib.lib().wam_linear_workspace_bytes(M, N, len(ws), K)
     if nbytes > 0:
-        # fp32 partial sums of the split-K tail
+        # fp32 partial sums of k ranges (freed to the stream that uses them:
+        # both are the current one)
         scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = scratch.data_ptr(), nbytes
     _lib.check(_lib.lib().wam_linear(ctypes.byref(a), stream_handle(dev)), "wam_linear")
-    if scratch is not None:
-        scratch.record_stream(torch.cuda.current_stream(dev))
     res = outs[0] if single else outs
     if mx_out:
         return res, mx_scale
@@ -378,15 +384,13 @@ def attention(q, k, v, *, pool_k=None, pool_v=None, slots=None, n_hist=None, poo
         a.q_ssq, a.q_ssq_n, a.q_norm_dim, a.q_eps = q_ssq.data_ptr(), q_ssq.shape[1], H * hd, q_eps
     # the key count bound plans the split: own keys plus the whole pool
     a.max_keys = a.Mk + (pool_k.shape[1] if n_hist is not None else 0)
-    ws = None
     nbytes = _lib.lib().wam_attention_workspace_bytes(a.B, a.Mq, a.H, a.max_keys)
     if nbytes > 0:
-        # partial results of the key-range splits
+        # partial results of the key-range splits (freed to the current
+        # stream, which uses them)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
     _lib.check(_lib.lib().wam_attention(ctypes.byref(a), stream_handle(dev)), "wam_attention")
-    if ws is not None:
-        ws.record_stream(torch.cuda.current_stream(dev))
     return o
 
 
