@@ -380,10 +380,8 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
   if (!split) WAM_TRY(qk_debug());
   // 3. q/k RMSNorm across heads + RoPE, in place.
   // 4. Pool bookkeeping: one workgroup's work, independent of the rows, so it
-  //    runs as a workgroup of the same launch (6240 slots: a launch of its own
-  //    took 9.5-11 us, 5 us read only; as a workgroup of the row pass 0.8-1.3
-  //    us of 2 x 16 rows, within the pass from 224 rows on).  Pools whose
-  //    flags do not fit 32 slots per thread of that launch keep their own.
+  //    runs as a workgroup of the same launch where that is no slower than a
+  //    launch of its own (kv_layout_rides).
   wam_kv_layout_args k{};
   if (cache) {
     k.mask = a->cache_mask; k.ids = a->cache_id; k.is_pred = a->cache_is_pred; k.pool = a->pool;
@@ -391,7 +389,7 @@ static int block_forward(const wam_block_args* a, hipStream_t s) {
     k.rows = a->candidate_rows; k.batch = B; k.pool_batch = a->cache_batch;
     k.hist_slots = slots; k.new_slots = newslots; k.info = info;
   }
-  const bool kv_rides = cache && a->pool <= kLayoutSlots * 256;
+  const bool kv_rides = cache && kv_layout_rides(a->pool, candidate);
   if (kv_rides) WAM_TRY(kv_layout_check(&k));
   {
     Scope sc(a->timer, WAM_STAGE_RMS_ROPE, s);

@@ -408,7 +408,7 @@ int rms_rope_check(const wam_rms_rope_args* a) {
 }
 
 // kv (may be null): the KV pool's bookkeeping, done by one workgroup of the
-// launch (pools of up to kLayoutSlots * 256 slots).
+// launch (where kv_layout_rides).
 int rms_rope(const wam_rms_rope_args* a, const wam_kv_layout_args* kv, hipStream_t s) {
   WAM_TRY(rms_rope_check(a));
   if (a->rows == 0) return WAM_OK;
