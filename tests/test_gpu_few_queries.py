@@ -163,25 +163,33 @@ def test_own_row_map_and_query_rms(dev):
     assert_close(ops.attention(q, k[:1], v[:1], q_ssq=ssq), ref, 2e-2, 0.9999, "query RMS factor")
 
 
-@pytest.mark.parametrize("B,Mq,Mk", [(1, 16, 6000), (1, 48, 3000)])
-def test_workspace_sizes(dev, B, Mq, Mk):
-    """No workspace, one short of the plan's, the plan's, and the entry point
-    without allocation: the same call, in as many ranges as fit."""
+# Workgroups of 32 and of 64 queries.  With 48 queries the general kernel is
+# the faster one once all of its own 32 ranges fit.
+@pytest.mark.parametrize("Mq,Mk,block,most", [(16, 6000, 32, 8), (48, 3001, 64, 32)])
+def test_workspace_sizes(dev, Mq, Mk, block, most):
+    """The same call with less and less room: no workspace, one byte less than
+    two ranges' partial results take, two and three ranges', one byte less
+    than all eight ranges', all, and what the size query asks for.  Ranges
+    that fit are used, nothing is written past them; the entry point without
+    allocation computes what the whole workspace gives."""
     from wam_ops import _lib
     H = 24
-    q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, Mk, H, 128), dev, 2), _randn((B, Mk, H, 128), dev, 3)
+    q, k, v = _randn((1, Mq, H, 128), dev, 1), _randn((1, Mk, H, 128), dev, 2), _randn((1, Mk, H, 128), dev, 3)
     ref = _ref(q, k, v, list(zip(k, v)))
     h = _lib.lib()
-    need = h.wam_attention_workspace_bytes(B, Mq, H, Mk)
-    assert need > 0
-    ws = torch.empty(need, dtype=torch.uint8, device=dev)
-    outs = []
-    for nbytes in (0, need - 1, need, None):
+    need = h.wam_attention_workspace_bytes(1, Mq, H, Mk)
+    # a range: per head and query of a workgroup 128 sums, a maximum and a weight
+    one = H * block * 130 * 4
+    assert need >= 8 * one
+    outs = {}
+    for nbytes, ranges in ((0, 1), (2 * one - 1, 1), (2 * one, 2), (4 * one - 1, 3), (8 * one - 1, 7), (8 * one, 8),
+                           (need, most), (None, None)):
+        ws = torch.full((max(need, 8 * one) + 4096,), 0xA5, dtype=torch.uint8, device=dev)
         o = torch.zeros_like(q)
         a = _lib.AttentionArgs()
         a.q, a.q_bstride, a.q_rstride = q.data_ptr(), q.stride(0), q.stride(1)
         a.o, a.o_bstride, a.o_rstride = o.data_ptr(), o.stride(0), o.stride(1)
-        a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch, a.scale, a.max_keys = B, Mq, H, 128, Mk, B, 128 ** -0.5, Mk
+        a.B, a.Mq, a.H, a.head_dim, a.Mk, a.kv_batch, a.scale, a.max_keys = 1, Mq, H, 128, Mk, 1, 128 ** -0.5, Mk
         a.k, a.v, a.kv_bstride, a.kv_rstride = k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1)
         if nbytes:
             a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
@@ -189,8 +197,14 @@ def test_workspace_sizes(dev, B, Mq, Mk):
         _lib.check(f(ctypes.byref(a), None), "wam_attention")
         torch.cuda.synchronize()
         assert_close(o, ref, 2e-2, 0.9999, f"workspace of {nbytes} bytes")
-        outs.append(o)
-    assert torch.equal(outs[2], outs[3])
+        outs[nbytes] = o
+        if nbytes is not None:
+            written = (ws != 0xA5).nonzero()
+            end = int(written[-1]) + 1 if written.numel() else 0
+            # (between two and what fits, the plan may find fewer as fast)
+            assert one < end <= ranges * one if ranges > 1 else end == 0, (nbytes, ranges, end / one)
+            assert ranges in (1, 7) or end > (ranges - 1) * one, (nbytes, ranges, end / one)
+    assert torch.equal(outs[need], outs[None]) and (most > 8 or torch.equal(outs[need], outs[8 * one]))
 
 
 # Few keys, where the two kernels' predicted times are close: own keys only,
