@@ -167,7 +167,7 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
     _req(not mx_out or (x8 and not xmx and single and out is None), "mx_out needs fp8 x with x_scale, one weight")
     _req(x.dim() >= 2 and x.stride(-1) == 1, "x must have a contiguous last dim")
     K = x.shape[-1]
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     M = x2.shape[0]
     N = ws[0].shape[0]
     for i, (w, b) in enumerate(zip(ws, bs)):
@@ -177,23 +177,27 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
                  "w_scale must be [N] fp32")
         else:
             _bf16(w, "weight")
-        _req(w.is_contiguous() and w.shape == (N, K), f"weight must be [{N}, {K}] contiguous")
+        if not w.is_contiguous() or w.shape != (N, K):
+            raise RuntimeError(f"weight must be [{N}, {K}] contiguous")
         if b is not None:
             _bf16(b, "bias")
             _req(b.is_contiguous() and b.numel() == N, "bias must be [N]")
     if mx_out:
         out_dtype = FP8
-    outs = out if out is not None else [torch.empty(*x.shape[:-1], N, dtype=out_dtype, device=dev)
-                                        for _ in ws]
-    if torch.is_tensor(outs):
-        outs = [outs]
+    if out is None:
+        shape = (M, N) if x2 is x else (*x.shape[:-1], N)
+        outs = [torch.empty(shape, dtype=out_dtype, device=dev) for _ in ws]
+    else:
+        outs = [out] if torch.is_tensor(out) else out
+        for o in outs[:len(ws)]:
+            _req(o.is_contiguous() and o.numel() == M * N and o.dtype == out_dtype, "out shape/dtype")
     a = _lib.LinearArgs()
     a.a, a.lda, a.M, a.K = x2.data_ptr(), x2.stride(0), M, K
     a.n_seg, a.seg_n, a.ldw = len(ws), N, K
     for i, (w, b, o) in enumerate(zip(ws, bs, outs)):
-        _req(o.is_contiguous() and o.numel() == M * N and o.dtype == out_dtype, "out shape/dtype")
         a.w[i] = w.data_ptr()
-        a.bias[i] = b.data_ptr() if b is not None else None
+        if b is not None:
+            a.bias[i] = b.data_ptr()
         a.out[i] = o.data_ptr()
     a.ldo = N
     a.epilogue = epilogue
@@ -245,13 +249,14 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
         _req(table is not None and temb is not None and gate_index is not None, "gate needs table/temb")
         a.gate = modulation(table, temb, tokens if tokens is not None else M)
         a.gate_index = gate_index
-    nbytes = _lib.lib().wam_linear_workspace_bytes(M, N, len(ws), K)
+    h = _lib.lib()
+    nbytes = h.wam_linear_workspace_bytes(M, N, len(ws), K)
     if nbytes > 0:
         # fp32 partial sums of k ranges (freed to the stream that uses them:
         # both are the current one)
         scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = scratch.data_ptr(), nbytes
-    _lib.check(_lib.lib().wam_linear(ctypes.byref(a), stream_handle(dev)), "wam_linear")
+    _lib.check(h.wam_linear(ctypes.byref(a), stream_handle(dev)), "wam_linear")
     res = outs[0] if single else outs
     if mx_out:
         return res, mx_scale
