@@ -149,6 +149,44 @@ def test_scales_not_above_zero(dev, scale, B, n, own):
     assert_close(ops.attention(q, k, v, scale=scale, **kw), ref, 2e-2, 0.9999, f"scale {scale}, {B}x{Mq}")
 
 
+# Rows of two and three pool rows, in equal shares: one workgroup per row, pairs
+# and ranges, threes and fours, pairs that straddle two pool rows.
+@pytest.mark.parametrize("B,Bp,Mq,n", [(10, 2, 16, 1300), (8, 2, 16, 5000), (6, 2, 5, 3000), (8, 2, 5, 2500), (9, 3, 10, 700),
+                                       (14, 2, 16, 400)])
+def test_shares_of_pool_rows(dev, B, Bp, Mq, n):
+    from wam_ops import ops
+    H = 24
+    q, k, v = _randn((B, Mq, H, 128), dev, 1, 2.0), _randn((B, Mq, H, 128), dev, 2), _randn((B, Mq, H, 128), dev, 3)
+    kw = _pool(dev, Bp, n + 3, H, torch.arange(n, device=dev), 4)
+    kw["pool_rows"] = torch.arange(B, device=dev) * Bp // B
+    src = [(torch.cat([kw["pool_k"][r, :n], k[b]]), torch.cat([kw["pool_v"][r, :n], v[b]]))
+           for b, r in enumerate(kw["pool_rows"].tolist())]
+    assert_close(ops.attention(q, k, v, **kw), _ref(q, k, v, src), 2e-2, 0.9999, f"{B} rows of {Bp} x {Mq} over {n}")
+
+
+def test_groups_do_not_straddle_pool_rows(dev):
+    """Ten rows over two pool rows take little more time than seven over one
+    (1.2 times; in pairs, one of which reads both pool rows, it was 2)."""
+    from wam_ops import ops
+    H, Mq, n = 24, 16, 1317
+    us = {}
+    for B, Bp in ((7, 1), (10, 2)):
+        q, k, v = _randn((B, Mq, H, 128), dev, 1), _randn((B, Mq, H, 128), dev, 2), _randn((B, Mq, H, 128), dev, 3)
+        kw = _pool(dev, Bp, n + 16, H, torch.arange(n, device=dev), 4)
+        kw["pool_rows"] = torch.arange(B, device=dev) * Bp // B
+        times = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                ops.attention(q, k, v, **kw)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 50)
+        us[B] = min(times)
+    assert us[10] < 1.55 * us[7], us
+
+
 def test_own_row_map_and_query_rms(dev):
     """kv_rows, and q_ssq's per-query factor (rows of the folded batch too)."""
     from wam_ops import ops

@@ -1137,9 +1137,10 @@ int64_t attention_workspace_bytes(int B, int Mq, int H, int64_t max_keys) {
     const FewPlan p = attention_few_plan(b, m, H, max_keys, sharing, INT64_MAX);
     if (p.qw) most = std::max(most, attention_few_bytes(p, b, m, H));
   };
-  few(B, Mq, 1);
-  for (int g = 2; g <= kFewGroupMax && g * (int64_t)Mq <= 32; ++g)
-    if (B % g == 0) few(B, Mq, g);
+  // (every count of batch rows per pool row that B / pool_batch takes; rows of
+  // more than 16 queries, or too many of them, are not grouped)
+  const bool groups = Mq <= 16 && B <= kFewGroupMax * device_cu_count();
+  for (int pb = groups ? 1 : B; pb >= 1 && pb <= B; pb = B / (B / pb) + 1) few(B, Mq, B / pb);
   if (B > 1 && (int64_t)B * Mq < (1 << 26)) few(1, B * Mq, 1);
   return most;
 }

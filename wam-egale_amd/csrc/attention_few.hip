@@ -396,30 +396,43 @@ int64_t attention_few_bytes(const FewPlan& p, int B, int Mq, int H) {
 //   2 x 128, 512 shared        20.2 -> 11.1     780, 780 keys       36 -> 24
 //   1024 (12 heads), 1024      28.3 -> 19.9     780, 512            31 -> 18
 //   16, 6016 keys (8 ranges)   28.4 -> 19.7     1560, 512           22 -> 35 (not taken)
-// Rows of one pool row are grouped as far as a wave's 32 queries: 14 x 16 in
-// groups of 2 is 168 workgroups with full waves (33 -> 27 us); groups of 7 on
-// four query waves, in 5 ranges, took the same time.
+// Batch rows of one pool row may be grouped as far as a wave's 32 queries
+// (g divides B), which reads their history once and leaves CUs for more
+// workgroups or key ranges.  A group that straddles two pool rows (g does not
+// divide the rows per pool row: 7 in pairs) has twice the history, and the
+// masks of other rows' keys make a round 2.3 us instead of 2: one workgroup
+// per row where that fits a dispatch round and the keys are not many.  16
+// queries a row, 24 heads, all slots valid (us: in pairs, one by one, and the
+// 256-query units):
+//   8 rows of 2, 1333 slots   24.9  20.1  31.8     10 rows of 2, 1333  33.3  20.1  32.0
+//   8 rows of 2, 6000 slots   53.4  61.8 113       4 rows of 1, 6000   29.4  37.0  74.4
+//   14 rows of 2, 1168 slots  30 (336 rows x heads do not fit one by one)
+// Plans go by the pool's slots, whatever is valid of them: over 16 valid ones
+// of 1333 one by one takes 7.2 us, in pairs 8.8, the units 5.9, and ranges,
+// whose merge does not depend on the keys, 13.6 (8 rows of 2, 3000 slots);
+// from a third of the slots on all of these are faster than the units.
 FewPlan attention_few_plan(int B, int Mq, int H, int64_t keys, int sharing, int64_t max_bytes) {
   const int cus = device_cu_count();
   FewPlan best{0, 1, 1, 1e30};
   if (B < 1 || Mq < 1 || B > (1 << 20) || Mq > 128 * cus || keys > (1 << 24)) return best;
-  int group = 1;
-  for (int g = 2; g <= kFewGroupMax && g <= sharing && g * Mq <= 32; ++g)
-    if (B % g == 0) group = g;
   const int tiles = (int)((keys + kFewKeys - 1) / kFewKeys);
   for (int qw = 1; qw <= 4; qw *= 2) {
-    const int g = qw == 1 ? group : 1;
-    const int64_t units = few_units(qw, g, B, Mq, H);
-    if (units > cus || (qw > 1 && Mq <= 16 * qw)) continue;
-    for (int r = 1; r <= kFewMaxRanges && units * r <= cus; ++r) {
-      if (r > 1 && r * kFewWaves / qw > tiles) break;
-      const FewPlan p{qw, g, r, 0};
-      const int64_t bytes = attention_few_bytes(p, B, Mq, H);
-      if (bytes > max_bytes) break;
-      const int rounds = ((tiles + r - 1) / r + kFewWaves / qw - 1) / (kFewWaves / qw);
-      const double per = qw == 4 ? 1.16 : (qw == 2 ? 1.45 : 2.0);
-      const double cost = 8.3 + (g > 1 ? 1.0 : 0.0) + rounds * per + (r > 1 ? 6.0 + 0.45e-6 * (double)bytes : 0.0);
-      if (cost < best.cost - 1e-9) best = FewPlan{qw, g, r, cost};
+    if (qw > 1 && Mq <= 16 * qw) continue;
+    for (int g = 1; g == 1 || (qw == 1 && g <= kFewGroupMax && g <= sharing && g * Mq <= 32); ++g) {
+      const int64_t units = few_units(qw, g, B, Mq, H);
+      if (B % g != 0 || units > cus) continue;
+      // the largest group's tiles (own rows of few keys: a tile each)
+      const int most = g > 1 ? tiles * (sharing % g != 0 ? 2 : 1) + g - 1 : tiles;
+      const double per = qw == 4 ? 1.16 : (qw == 2 ? 1.45 : (g > 1 ? 2.3 : 2.0));
+      for (int r = 1; r <= kFewMaxRanges && units * r <= cus; ++r) {
+        if (r > 1 && r * kFewWaves / qw > tiles) break;
+        const FewPlan p{qw, g, r, 0};
+        const int64_t bytes = attention_few_bytes(p, B, Mq, H);
+        if (bytes > max_bytes) break;
+        const int rounds = ((most + r - 1) / r + kFewWaves / qw - 1) / (kFewWaves / qw);
+        const double cost = 8.3 + (g > 1 ? 1.0 : 0.0) + rounds * per + (r > 1 ? 6.0 + 0.45e-6 * (double)bytes : 0.0);
+        if (cost < best.cost - 1e-9) best = FewPlan{qw, g, r, cost};
+      }
     }
   }
   return best;
