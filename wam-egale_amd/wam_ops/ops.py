@@ -167,8 +167,12 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
     _req(not mx_out or (x8 and not xmx and single and out is None), "mx_out needs fp8 x with x_scale, one weight")
     _req(x.dim() >= 2 and x.stride(-1) == 1, "x must have a contiguous last dim")
     K = x.shape[-1]
-    x2 = x if x.dim() == 2 else x.reshape(-1, K)
-    M = x2.shape[0]
+    if x.dim() > 2 and K > 0 and x.is_contiguous():
+        M, lda = x.numel() // K, K
+        x2 = x
+    else:
+        x2 = x if x.dim() == 2 else x.reshape(-1, K)
+        M, lda = x2.shape[0], x2.stride(0)
     N = ws[0].shape[0]
     for i, (w, b) in enumerate(zip(ws, bs)):
         if f8:
@@ -185,14 +189,14 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
     if mx_out:
         out_dtype = FP8
     if out is None:
-        shape = (M, N) if x2 is x else (*x.shape[:-1], N)
+        shape = (M, N) if x.dim() == 2 else (*x.shape[:-1], N)
         outs = [torch.empty(shape, dtype=out_dtype, device=dev) for _ in ws]
     else:
         outs = [out] if torch.is_tensor(out) else out
         for o in outs[:len(ws)]:
             _req(o.is_contiguous() and o.numel() == M * N and o.dtype == out_dtype, "out shape/dtype")
     a = _lib.LinearArgs()
-    a.a, a.lda, a.M, a.K = x2.data_ptr(), x2.stride(0), M, K
+    a.a, a.lda, a.M, a.K = x2.data_ptr(), lda, M, K
     a.n_seg, a.seg_n, a.ldw = len(ws), N, K
     for i, (w, b, o) in enumerate(zip(ws, bs, outs)):
         a.w[i] = w.data_ptr()
@@ -242,7 +246,7 @@ def linear(x, weights, biases=None, *, epilogue=EPI_BIAS, residual=None, table=N
             a.norm_head_dim = norm_head_dim
     if epilogue in (EPI_BIAS_GATE_RES, EPI_BIAS_RES):
         _req(residual is not None, "residual required")
-        r2 = residual.reshape(-1, N)
+        r2 = residual if residual.shape == (M, N) else residual.reshape(-1, N)
         _req(r2.shape[0] == M and r2.stride(-1) == 1, "residual must be [M, N]")
         a.res, a.ldr, a.res_dtype = r2.data_ptr(), r2.stride(0), dtype_code(r2)
     if epilogue == EPI_BIAS_GATE_RES:
