@@ -484,7 +484,12 @@ int wam_rope_freqs(const wam_rope_freq_args* args, void* stream);
 
 /* --------------------------------------------------------------- timing */
 /* Stage timer: pairs of HIP events recorded on the launch stream around
- * selected stages of wam_block_forward. */
+ * selected stages of wam_block_forward.  Work that runs inside another
+ * stage's launch counts there, and its own stage then times nothing: the
+ * pool's bookkeeping (KV_LAYOUT) in RMS_ROPE for pools of up to 4096 slots,
+ * 8192 read only; with few rows (a projection split over k) the commit
+ * (KV_COMMIT) in LN2, and the reductions, biases and residuals of QKV, SELF_OUT
+ * and CROSS_OUT in RMS_ROPE, LN2 and LN3. */
 enum {
   WAM_STAGE_LN1 = 0, WAM_STAGE_QKV, WAM_STAGE_RMS_ROPE, WAM_STAGE_KV_LAYOUT,
   WAM_STAGE_SELF_ATTN, WAM_STAGE_SELF_OUT, WAM_STAGE_LN2, WAM_STAGE_CROSS_Q,
